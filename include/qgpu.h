@@ -183,6 +183,34 @@ int  qgpu_add_partials(float *y, uint64_t ldy, const float *x, uint64_t ldx, con
 int  qgpu_gemv_rows_batch(const qgpu_tensor *W, const float *x, uint64_t ldx, int n,
                           float *out, uint64_t ldo, uint64_t r0, uint64_t r1);
 
+/* ------------------------------------------------------------ prompt products */
+/* Products of a matrix with many rows (tokens) at once, for prompts: no reference counterpart (its
+ * prefill calls gemv_batch on 8 tokens at a time).  A workspace holds the prepared rows:
+ * qgpu_wide_prepare converts act's rows (QGPU_ACT_* without pending planes, gather or xout; a
+ * gated norm has heads of 128; x, y, w, w2 16-byte aligned, ldx and ldy multiples of 4) and
+ * qgpu_wide_gemm multiplies them, out[t*ldo + r] (+)= sum_i W[r,i] v[t][i], with every matrix of
+ * the call (matrix-core formats only: qgpu_wide_supports).  n <= max_rows, ne0 <= max_k.
+ * n_ctx positions of n_kv heads and n_k / n_v GDN heads size the workspaces of qgpu_wide_attn and
+ * qgpu_wide_gdn (0: those calls are rejected). */
+typedef struct qgpu_wide qgpu_wide;
+int  qgpu_wide_create(int max_rows, uint64_t max_k, int n_ctx, int n_kv, int n_k, int n_v, qgpu_wide **out);
+int  qgpu_wide_free(qgpu_wide *w);
+int  qgpu_wide_supports(const qgpu_tensor *W);
+int  qgpu_wide_prepare(qgpu_wide *w, const qgpu_act *act, int n, uint64_t ne0);
+int  qgpu_wide_gemm(qgpu_wide *w, const qgpu_tensor *const *Ws, int n_mat, int n, float *const *outs,
+                    const uint64_t *ldos, int flags);
+/* qgpu_attn_decode for n tokens at positions pos..pos+n-1 (q prepared and the caches written by
+ * qgpu_attn_prep); pos + n <= n_ctx, n_kv as created. */
+int  qgpu_wide_attn(qgpu_wide *w, const float *q, uint64_t ldq, const float *kcache, const float *vcache,
+                    int pos, int n, int n_head, int n_kv, int head_dim, float *out, uint64_t ldo);
+/* qgpu_gdn_fused for n tokens without the snapshots in between: the conv window and the state before
+ * the first token are read from conv_in and ssm_in, those after the last one written to conv_out and
+ * ssm_out (other memory). */
+int  qgpu_wide_gdn(qgpu_wide *w, const float *x, uint64_t ldx, int n, const float *conv_w, const float *conv_in,
+                   float *conv_out, const float *beta_raw, const float *alpha_raw, uint64_t ldba,
+                   const float *dt_bias, const float *ssm_a, const float *ssm_in, float *ssm_out, int n_k, int n_v,
+                   int head_dim, float eps, float *out, uint64_t ldo);
+
 /* ------------------------------------------------------------ dequant */
 /* out[b*ldo + i] = dequant(row rows[b])[i] for b < n, rows in DEVICE memory.
  * Bit-exact with the reference scalar decoder (quant.c:86-208); replaces the

@@ -17,7 +17,7 @@ enum { T_F32 = 0, T_F16 = 1, T_Q8_0 = 8, T_Q4_K = 12, T_Q5_K = 13, T_Q6_K = 14, 
 #define IQ4_TILE_ROWS   16
 #define IQ4_REC_BYTES   2176
 #define IQ4_HDR_BYTES   128
-static inline __host__ __device__ uint32_t packed_rec_bytes(int type)
+static inline __host__ __device__ constexpr uint32_t packed_rec_bytes(int type)
 {
     switch (type) {
     case T_IQ4_XS: return 2176;
@@ -204,6 +204,18 @@ static __device__ __forceinline__ void tok_digits(float v, float mx, int i, uint
     if (c < 3) *(uint32_t *)(tile + ((lane >> 2) & 3) * 48 + c * 16 + (lane >> 4) * 4) = W;
     if (e < 4) xs_tile[4 * e + i] = ldexpf(1.0f, 8 * e - shift);
 }
+
+// Workspace of the prompt path (wide.hip, wide_seq.hip).
+struct qgpu_wide {
+    int rows;                           // tokens it holds (a multiple of 128)
+    uint64_t max_k;
+    uint8_t *A, *S;                     // prepared activations: hi and lo planes, sub-block sums
+    float *xs, *piece;                  // row scales; partial results of tiles shared by blocks
+    int n_ctx, n_kv;
+    uint8_t *kv;                        // K and V operands of n_ctx positions (32-position tiles)
+    int gdn_heads, gdn_chan;
+    float *y, *gate;                    // GDN: convolved channels (gdn_chan heads of 128), gates (gdn_heads rows)
+};
 
 namespace qg {
 extern hipStream_t stream;

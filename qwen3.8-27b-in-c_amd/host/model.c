@@ -25,6 +25,11 @@
 
 #define NSLOT (SPEC_MAX_B + 1)      /* GDN state ring: current + one snapshot per batch token */
 #define MAXB  SPEC_MAX_B
+#define WIDE_ROWS 2048              /* prompt tokens per wide chunk at most (a multiple of 8) */
+/* Prompt tokens before the last batch from which the wide path is taken.  Measured at the 27B layer shapes, 8
+ * layers, a prompt's ingestion: 16 such tokens 2.67 ms in batches of 8 and 2.72 ms wide (mixed formats
+ * 2.52 and 2.59), 24 tokens 3.62 and 2.74 ms (3.36 and 2.60). */
+#define WIDE_MIN  24
 
 double qwen_prof_embed, qwen_prof_gdn, qwen_prof_attn, qwen_prof_head;
 uint64_t qwen_prof_calls;
@@ -86,6 +91,11 @@ struct qwen_gpu {
      * (kind, token pointer, hidden-state pointer, logits pointer, B, flag, att_live) */
     int use_graphs, n_graphs;
     struct { int kind, flag, live; uint32_t B; const void *tok, *h, *lg; void *exec; } graphs[48];
+    /* wide prompt path (prefill_wide): workspace and fp32 rows of up to w_rows tokens; NULL when a
+     * matrix of the model has no matrix-core form (the prompt then goes in batches of 8 throughout) */
+    qgpu_wide *wide;
+    uint32_t w_rows, *w_tok;
+    float *wx, *wa, *wb, *wo, *wk, *wv, *wbeta, *walpha;
     int status;               /* of the last call: 0, -1 rejected on the host, -2 device error */
     /* section timing of model_forward: events before the embedding, after it, after each layer
      * and after the head (n_layer + 3), recorded while prof_active */
@@ -166,6 +176,7 @@ static void gpu_free(qwen_gpu_t *g)
             if (g->pev[i]) qgpu_event_destroy(g->pev[i]);
         free(g->pev);
     }
+    qgpu_wide_free(g->wide);
     for (size_t i = 0; i < g->n_tensors; i++) qgpu_tensor_free(g->tensors[i]);
     for (size_t i = 0; i < g->n_allocs; i++) qgpu_free(g->allocs[i]);
     qgpu_host_free(g->h_acc);
@@ -303,6 +314,39 @@ static int upload_layer(qwen_gpu_t *g, const source_t *src, const qwen_layer_t *
             !(D->q_norm = up_f32(g, src, L->attn_q_norm)) || !(D->k_norm = up_f32(g, src, L->attn_k_norm)))
             return -1;
     }
+    return 0;
+}
+
+/* workspace of the wide prompt path, when every matrix it multiplies runs on the matrix cores */
+static int wide_init(qwen_model_t *m)
+{
+    qwen_gpu_t *g = m->gpu;
+    const qwen_dims_t *d = &m->dims;
+    const uint64_t E = d->n_embd, F = d->n_ff, hd = (uint64_t)d->n_head * d->head_dim;
+    for (uint32_t il = 0; il <= d->n_layer; il++) {
+        const glayer_t *D = il < d->n_layer ? &g->L[il] : &g->mtp;
+        const qgpu_tensor *W[] = { D->ffn_gate, D->ffn_up, D->ffn_down, D->rec ? D->wqkv : D->q,
+                                   D->rec ? D->wgate : D->k, D->rec ? D->beta : D->v, D->rec ? D->alpha : D->o,
+                                   D->rec ? D->ssm_out : D->o };
+        for (size_t i = 0; i < sizeof W / sizeof *W; i++)
+            if (!qgpu_wide_supports(W[i])) return 0;
+    }
+    if (!qgpu_wide_supports(g->eh_proj) || d->n_v_heads % d->n_k_heads) return 0;
+    uint64_t K = F > 2 * E ? F : 2 * E;
+    if (g->A > K) K = g->A;
+    const uint32_t R = m->n_ctx < WIDE_ROWS ? (m->n_ctx + 7) / 8 * 8 : WIDE_ROWS;
+    if (qgpu_wide_create((int)R, K, (int)m->n_ctx, (int)d->n_kv_head, (int)d->n_k_heads, (int)d->n_v_heads, &g->wide))
+        return -1;
+    g->w_rows = R;
+    const uint64_t B2 = F > E ? F : E, wb = B2 > d->d_inner ? B2 : d->d_inner;
+    uint64_t wa = d->conv_dim > 2 * hd ? d->conv_dim : 2 * hd;
+    if (F > wa) wa = F;
+    if (E > wa) wa = E;
+#define AL(p, n) do { if (!((p) = dalloc(g, (n) * sizeof(*(p))))) return -1; } while (0)
+    AL(g->w_tok, R); AL(g->wx, R * E); AL(g->wa, R * wa); AL(g->wb, R * wb); AL(g->wo, R * g->A);
+    AL(g->wk, R * g->kvrow); AL(g->wv, R * g->kvrow);
+    AL(g->wbeta, R * (uint64_t)d->n_v_heads); AL(g->walpha, R * (uint64_t)d->n_v_heads);
+#undef AL
     return 0;
 }
 
@@ -481,7 +525,7 @@ static int model_load(qwen_model_t *m, const source_t *src, uint32_t n_ctx)
               qgpu_memcpy_h2d(g->rope_sin, sn, (size_t)n_ctx * half * sizeof(float)));
     m->rope_cos = cs;                          /* host copies (reference field names) */
     m->rope_sin = sn;
-    if (rc || qgpu_attn_reserve((int)n_ctx, (int)d->n_kv_head)) return -1;
+    if (rc || qgpu_attn_reserve((int)n_ctx, (int)d->n_kv_head) || wide_init(m)) return -1;
     for (int b = 1; b <= QGPU_MAX_B; b++)
         g->att_split[b] = qgpu_attn_split_bound((int)n_ctx, b, (int)d->n_head, (int)d->n_kv_head);
     /* host-side fields, laid out as the reference's arenas (model.c:166-230) */
@@ -1175,11 +1219,130 @@ void gdn_layer(qwen_model_t *m, qwen_layer_t *L, pool_t *pool)
 }
 
 /* ------------------------------------------------------------------ device-resident generation */
+/* Wide prompt path: chunks of up to w_rows tokens go through every matrix in one product
+ * (qgpu_wide_gemm), the layers' token mixing in one launch sequence (qgpu_wide_gdn, qgpu_wide_attn).
+ * It leaves what the tokens after it read: the KV caches (the MTP layer's too), the GDN states (in
+ * ring slot cur) and nothing else; prefill_dev runs the prompt's last batch on the ordinary path, so
+ * logits, hidden rows and rollback states are those of a batch as before. */
+static void wide_mul(qwen_model_t *m, const qgpu_act *act, uint32_t M, const qgpu_tensor *const *W, int n_mat,
+                     float *const *outs, const uint64_t *ld, int flags)
+{
+    int t;
+    uint64_t ne0 = 0, ne1;
+    K(qgpu_tensor_shape(W[0], &t, &ne0, &ne1));
+    K(qgpu_wide_prepare(m->gpu->wide, act, (int)M, ne0));
+    K(qgpu_wide_gemm(m->gpu->wide, W, n_mat, (int)M, outs, ld, flags));
+}
+
+static qgpu_act act_rows(int kind, const float *x, uint64_t ldx)
+{
+    qgpu_act a;
+    memset(&a, 0, sizeof a);
+    a.kind = kind; a.x = x; a.ldx = ldx;
+    return a;
+}
+
+static void wide_ffn(qwen_model_t *m, const glayer_t *D, uint32_t M)
+{
+    qwen_gpu_t *g = m->gpu;
+    const uint64_t E = m->dims.n_embd, F = m->dims.n_ff;
+    const qgpu_tensor *W[2] = { D->ffn_gate, D->ffn_up };
+    float *outs[2] = { g->wa, g->wb };
+    const uint64_t ld[2] = { F, F };
+    const qgpu_act an = act_norm(g->wx, E, D->post_norm, m->cfg.rms_norm_eps, NULL, 0);
+    wide_mul(m, &an, M, W, 2, outs, ld, 0);
+    qgpu_act sm = act_rows(QGPU_ACT_SILU_MUL, g->wa, F);
+    sm.y = g->wb; sm.ldy = F;
+    wide_mul(m, &sm, M, (const qgpu_tensor *const *)&D->ffn_down, 1, &g->wx, &E, QGPU_GEMV_ACCUM);
+}
+
+/* kv_only: the layer's outputs are not read (the cache rows are) */
+static void wide_attn(qwen_model_t *m, const glayer_t *D, const float *x, uint32_t M, uint32_t pos, int kv_only)
+{
+    qwen_gpu_t *g = m->gpu;
+    const qwen_dims_t *d = &m->dims;
+    const uint64_t E = d->n_embd, ldq = 2ull * d->n_head * d->head_dim;
+    const float eps = m->cfg.rms_norm_eps;
+    const qgpu_tensor *W[3] = { D->k, D->v, D->q };
+    float *outs[3] = { g->wk, g->wv, g->wa };
+    const uint64_t ld[3] = { g->kvrow, g->kvrow, ldq };
+    const qgpu_act an = act_norm(x, E, D->attn_norm, eps, NULL, 0);
+    wide_mul(m, &an, M, W, kv_only ? 2 : 3, outs, ld, 0);
+    K(qgpu_attn_prep(g->wa, ldq, g->wk, g->wv, g->kvrow, D->q_norm, D->k_norm, D->kv_k, D->kv_v, g->rope_cos,
+                     g->rope_sin, (int)m->cfg.rope_dim_count, g->d_posv + pos, (int)M, kv_only ? 0 : (int)d->n_head,
+                     (int)d->n_kv_head, (int)d->head_dim, eps));
+    if (kv_only) return;
+    K(qgpu_wide_attn(g->wide, g->wa, ldq, D->kv_k, D->kv_v, (int)pos, (int)M, (int)d->n_head, (int)d->n_kv_head,
+                     (int)d->head_dim, g->wo, g->A));
+    const qgpu_act oc = act_rows(QGPU_ACT_COPY, g->wo, g->A);
+    wide_mul(m, &oc, M, (const qgpu_tensor *const *)&D->o, 1, &g->wx, &E, QGPU_GEMV_ACCUM);
+    wide_ffn(m, D, M);
+}
+
+static void wide_gdn(qwen_model_t *m, const glayer_t *D, uint32_t M, int from, int to, int state_only)
+{
+    qwen_gpu_t *g = m->gpu;
+    const qwen_dims_t *d = &m->dims;
+    const uint64_t E = d->n_embd, di = d->d_inner, nv = d->n_v_heads, cd = d->conv_dim;
+    const float eps = m->cfg.rms_norm_eps;
+    const qgpu_tensor *W[4] = { D->wqkv, D->wgate, D->beta, D->alpha };
+    float *outs[4] = { g->wa, g->wb, g->wbeta, g->walpha };
+    const uint64_t ld[4] = { cd, di, nv, nv };
+    const qgpu_act an = act_norm(g->wx, E, D->attn_norm, eps, NULL, 0);
+    wide_mul(m, &an, M, W, 4, outs, ld, 0);
+    K(qgpu_wide_gdn(g->wide, g->wa, cd, (int)M, D->conv1d, D->conv_ring + (size_t)from * g->conv_elems,
+                    D->conv_ring + (size_t)to * g->conv_elems, g->wbeta, g->walpha, nv, D->dt_bias, D->ssm_a,
+                    D->ssm_ring + (size_t)from * g->ssm_elems, D->ssm_ring + (size_t)to * g->ssm_elems,
+                    (int)d->n_k_heads, (int)d->n_v_heads, (int)d->head_v_dim, eps, g->wo, di));
+    if (state_only) return;
+    qgpu_act gn = act_rows(QGPU_ACT_GATED_NORM, g->wo, di);
+    gn.y = g->wb; gn.ldy = di; gn.w = D->ssm_norm; gn.seg = d->head_v_dim; gn.eps = eps;
+    wide_mul(m, &gn, M, (const qgpu_tensor *const *)&D->ssm_out, 1, &g->wx, &E, QGPU_GEMV_ACCUM);
+    wide_ffn(m, D, M);
+}
+
+static void prefill_wide(qwen_model_t *m, const uint32_t *prompt, uint32_t n, int with_mtp)
+{
+    qwen_gpu_t *g = m->gpu;
+    const qwen_dims_t *d = &m->dims;
+    const uint64_t E = d->n_embd;
+    gdn_settle(m);
+    for (uint32_t pos = 0; pos < n;) {
+        const uint32_t M = n - pos < g->w_rows ? n - pos : g->w_rows;
+        const int from = g->cur, to = (g->cur + 1) % NSLOT;
+        K(qgpu_memcpy_h2d(g->w_tok, prompt + pos, M * sizeof(uint32_t)));
+        K(qgpu_dequant_rows(g->tok_embd, g->w_tok, (int)M, g->wx, E));
+        for (uint32_t il = 0; il < d->n_layer; il++) {
+            /* without the MTP layer nothing reads the last layer's rows, only its cache or state */
+            const int last = !with_mtp && il + 1 == d->n_layer;
+            if (g->L[il].rec) wide_gdn(m, &g->L[il], M, from, to, last);
+            else wide_attn(m, &g->L[il], g->wx, M, pos, last);
+        }
+        if (with_mtp) {
+            /* the MTP layer's cache rows: eh_proj(concat(enorm(e), hnorm(h))) and its k, v */
+            K(qgpu_dequant_rows(g->tok_embd, g->w_tok, (int)M, g->wb, E));
+            qgpu_act cat = act_norm(g->wb, E, g->enorm, m->cfg.rms_norm_eps, NULL, 0);
+            cat.y = g->wx; cat.ldy = E; cat.w2 = g->hnorm; cat.seg = E;
+            wide_mul(m, &cat, M, (const qgpu_tensor *const *)&g->eh_proj, 1, &g->wa, &E, 0);
+            wide_attn(m, &g->mtp, g->wa, M, pos, 1);
+        }
+        g->cur = g->cur_base = to;
+        g->fbase = -1;
+        g->last_B = 0;
+        pos += M;
+    }
+}
+
 /* returns the rows of the last chunk: the prompt's last logits row is logits_b[last - 1] */
 static uint32_t prefill_dev(qwen_model_t *m, const uint32_t *prompt, uint32_t n, int with_mtp)
 {
     qwen_gpu_t *g = m->gpu;
     uint32_t pos = 0, last = 0;
+    const uint32_t body = (n - 1) / PREFILL_MAX_B * PREFILL_MAX_B;        /* all but the last batch */
+    if (g->wide && body >= WIDE_MIN) {
+        prefill_wide(m, prompt, body, with_mtp);
+        pos = body;
+    }
     while (pos < n) {
         const uint32_t B = n - pos > PREFILL_MAX_B ? PREFILL_MAX_B : n - pos;
         put_tokens(m, prompt + pos, B);
