@@ -17,11 +17,6 @@
 // elements 4g..4g+3 and 16+4g..16+4g+3, the order in which the packed weight records hold
 // their lanes' dwords (gemv.hip), so a lane's nibble dword decodes straight into its B operand.
 //
-// What it gives: a 512-token prompt through eight layers of the 27B shapes 61.7 -> 12.3 ms, 1999 tokens with
-// the checkpoint's format mix 255 -> 38.5 ms.  The product of 5120 -> 34816 (IQ4_XS) runs at 462 TFLOP/s of
-// useful work at 1992 tokens (two half-precision products each; a library fp16 product of 8192^3 reaches
-// 1106 on the same card); against FP64 it is 1.2e-7 off, the GEMV path 6.4e-7.
-//
 // Schedule.  A block of 4 waves owns 16*MTL tokens x 256 weight rows (64 per wave: the
 // wave decodes its own weights in registers, and the activation tile is shared through LDS).  The
 // (tile, super-block) units of a launch are cut into equal contiguous runs, one per resident
@@ -78,16 +73,26 @@ static __device__ __forceinline__ uint32_t spread4(uint32_t x) { return (x * 0x0
 // ---------------------------------------------------------------- weight records
 // One lane's slice of a 16-row record, by halves of four sub-blocks: hdr() loads what the whole
 // super-block shares, half() the quants of one half; code(ib) decodes a sub-block's eight elements
-// to fp16 integers and scale(ib) gives its fp32 factor.
+// to fp16 integers and scale(ib) gives its fp32 factor.  Loads go through a buffer resource at the
+// wave's first tile: a scalar offset per record, one vector offset for all of them.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+static __device__ __forceinline__ uint4 ld128(rsrc_t rs, uint32_t vo, uint32_t so)
+{
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0));
+}
+static __device__ __forceinline__ uint2 ld64(rsrc_t rs, uint32_t vo, uint32_t so)
+{
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0));
+}
 template <int FMT> struct WideW;
 
 template <> struct WideW<T_IQ4_XS> {
     uint2 h;
     uint4 q;
-    __device__ __forceinline__ void hdr(const uint8_t *rec, int n) { h = *(const uint2 *)(rec + n * 8); }
-    __device__ __forceinline__ void half(const uint8_t *rec, int lane, int hf)
+    __device__ __forceinline__ void hdr(rsrc_t rs, uint32_t so, uint32_t l16) { h = ld64(rs, (l16 & 240) >> 1, so); }
+    __device__ __forceinline__ void half(rsrc_t rs, uint32_t so, uint32_t l16, int hf)
     {
-        q = *(const uint4 *)(rec + IQ4_HDR_BYTES + hf * 1024 + lane * 16);
+        q = ld128(rs, l16 + IQ4_HDR_BYTES + hf * 1024, so);
     }
     // codebook + 128 as one byte: two 8-entry v_perm_b32 tables indexed by the whole nibble, whose
     // out-of-range selectors give 0x00 or 0xFF and are undone in the other table (xor)
@@ -122,10 +127,10 @@ static __device__ __forceinline__ uint32_t kq_m(uint4 h, int ib)
 }
 template <> struct WideW<T_Q4_K> {
     uint4 h, q;
-    __device__ __forceinline__ void hdr(const uint8_t *rec, int n) { h = *(const uint4 *)(rec + n * 16); }
-    __device__ __forceinline__ void half(const uint8_t *rec, int lane, int hf)
+    __device__ __forceinline__ void hdr(rsrc_t rs, uint32_t so, uint32_t l16) { h = ld128(rs, l16 & 240, so); }
+    __device__ __forceinline__ void half(rsrc_t rs, uint32_t so, uint32_t l16, int hf)
     {
-        q = *(const uint4 *)(rec + 256 + hf * 1024 + lane * 16);
+        q = ld128(rs, l16 + 256 + hf * 1024, so);
     }
     __device__ __forceinline__ v8h code(int ib) const
     {
@@ -137,11 +142,11 @@ template <> struct WideW<T_Q4_K> {
 template <> struct WideW<T_Q5_K> {
     uint4 h, q;
     uint32_t hb;
-    __device__ __forceinline__ void hdr(const uint8_t *rec, int n) { h = *(const uint4 *)(rec + n * 16); }
-    __device__ __forceinline__ void half(const uint8_t *rec, int lane, int hf)
+    __device__ __forceinline__ void hdr(rsrc_t rs, uint32_t so, uint32_t l16) { h = ld128(rs, l16 & 240, so); }
+    __device__ __forceinline__ void half(rsrc_t rs, uint32_t so, uint32_t l16, int hf)
     {
-        q = *(const uint4 *)(rec + 256 + hf * 1024 + lane * 16);
-        hb = *(const uint32_t *)(rec + 2304 + lane * 8 + hf * 4);
+        q = ld128(rs, l16 + 256 + hf * 1024, so);
+        hb = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, (l16 >> 1) + 2304 + hf * 4, so, 0);
     }
     __device__ __forceinline__ v8h code(int ib) const
     {
@@ -155,15 +160,15 @@ template <> struct WideW<T_Q6_K> {
     uint4 h, q;
     uint2 hb;
     float d;
-    __device__ __forceinline__ void hdr(const uint8_t *rec, int n)
+    __device__ __forceinline__ void hdr(rsrc_t rs, uint32_t so, uint32_t l16)
     {
-        h = *(const uint4 *)(rec + n * 16);
-        d = h2f(*(const uint16_t *)(rec + 256 + 2 * n));
+        h = ld128(rs, l16 & 240, so);
+        d = h2f((uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, 256 + ((l16 & 240) >> 3), so, 0));
     }
-    __device__ __forceinline__ void half(const uint8_t *rec, int lane, int hf)
+    __device__ __forceinline__ void half(rsrc_t rs, uint32_t so, uint32_t l16, int hf)
     {
-        q = *(const uint4 *)(rec + 288 + hf * 1024 + lane * 16);
-        hb = *(const uint2 *)(rec + 2336 + lane * 16 + hf * 8);
+        q = ld128(rs, l16 + 288 + hf * 1024, so);
+        hb = ld64(rs, l16 + 2336 + hf * 8, so);
     }
     __device__ __forceinline__ v8h code(int ib) const
     {
@@ -179,11 +184,11 @@ template <> struct WideW<T_Q6_K> {
 };
 template <> struct WideW<T_Q8_0> {
     uint4 h, q[2];
-    __device__ __forceinline__ void hdr(const uint8_t *rec, int n) { h = *(const uint4 *)(rec + n * 16); }
-    __device__ __forceinline__ void half(const uint8_t *rec, int lane, int hf)
+    __device__ __forceinline__ void hdr(rsrc_t rs, uint32_t so, uint32_t l16) { h = ld128(rs, l16 & 240, so); }
+    __device__ __forceinline__ void half(rsrc_t rs, uint32_t so, uint32_t l16, int hf)
     {
-        q[0] = *(const uint4 *)(rec + 256 + ((2 * hf) * 64 + lane) * 16);
-        q[1] = *(const uint4 *)(rec + 256 + ((2 * hf + 1) * 64 + lane) * 16);
+        q[0] = ld128(rs, l16 + 256 + hf * 2048, so);
+        q[1] = ld128(rs, l16 + 256 + hf * 2048 + 1024, so);
     }
     __device__ __forceinline__ v8h code(int ib) const
     {
@@ -199,7 +204,12 @@ typedef const __attribute__((address_space(1))) void *gptr_t;
 typedef __attribute__((address_space(3))) void *lptr_t;
 
 // Stage: two sub-blocks of the block's activation tile (MTL * 4 KB), brought into one of two LDS
-// buffers by direct loads while the other is used; one barrier per stage.
+// buffers by direct loads while the other is used; one barrier per stage.  Bound by the matrix cores
+// (55% of their cycles at 1992 tokens) beside the multiply-adds and decoding on the vector units (49%).
+// Loads take scalar offsets from buffer resources, the next quants the registers of the ones just
+// decoded, and a row tile's multiply-adds run beside the next tile's products: 256 registers hold it, two
+// waves per SIMD.  5120 -> 34816 at 1992 / 256 tokens 1537 / 231 -> 1440 / 208 us, 17408 -> 5120 765 /
+// 140 -> 708 / 133 us, against per-lane addresses, copies of the next quants and no such overlap.
 template <int FMT, int MTL>
 __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
 {
@@ -215,6 +225,7 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
     uint32_t u = (uint32_t)((uint64_t)g * a.U / a.G);
     const uint32_t ue = (uint32_t)((uint64_t)(g + 1) * a.U / a.G);
     const uint64_t nsub = (uint64_t)a.nsb * 8;
+    const uint32_t l16 = (uint32_t)lane * 16;
     const v4f z4 = { 0.0f, 0.0f, 0.0f, 0.0f };
     while (u < ue) {
         const uint32_t tile = u / a.nsb, sb0 = u - tile * a.nsb, sb1 = min(a.nsb, sb0 + (ue - u));
@@ -222,39 +233,37 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
         int j = 0;
         while (j + 1 < a.n_mat && nt >= a.m[j + 1].tile0) j++;
         const uint32_t row0 = (nt - a.m[j].tile0) * WIDE_N + wv * (WIDE_NT * 16);   // this wave's first weight row
-        const uint64_t tstr = (uint64_t)a.nsb * REC;
-        const uint8_t *rec[WIDE_NT];
+        // its records: past the matrix's end any loadable one (the results are dropped)
+        const uint32_t tstr = a.nsb * REC, t0 = min(row0 / 16, a.m[j].nt16 - 1);
+        const rsrc_t rsW = __builtin_amdgcn_make_buffer_rsrc((void *)(a.m[j].W + (uint64_t)t0 * tstr), 0, 0x7FFFFFFF, 0x00020000);
+        uint32_t rec[WIDE_NT];
 #pragma unroll
-        for (int t = 0; t < WIDE_NT; t++) {
-            const uint32_t t16 = min(row0 / 16 + t, a.m[j].nt16 - 1);               // past the end: any loadable record
-            rec[t] = a.m[j].W + t16 * tstr + (uint64_t)sb0 * REC;
-        }
+        for (int t = 0; t < WIDE_NT; t++) rec[t] = min((uint32_t)t, a.m[j].nt16 - 1 - t0) * tstr + sb0 * REC;
         v4f acc[MTL][WIDE_NT];
 #pragma unroll
         for (int mt = 0; mt < MTL; mt++)
 #pragma unroll
             for (int t = 0; t < WIDE_NT; t++) acc[mt][t] = z4;
         // this wave's MTL 1 KB chunks of a stage: chunk c = (row tile c / 4, 1 KB part c % 4)
-        const uint8_t *Ag = a.A + ((uint64_t)mb * MTL * nsub + (uint64_t)sb0 * 8) * WIDE_SUB;
-        const uint32_t l16 = (uint32_t)lane * 16;
+        const rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(a.A + ((uint64_t)mb * MTL * nsub + (uint64_t)sb0 * 8) * WIDE_SUB), 0, 0x7FFFFFFF, 0x00020000);
         auto stage = [&](uint32_t s, uint8_t *buf) {
 #pragma unroll
             for (int i = 0; i < MTL; i++) {
                 const int c = wv * MTL + i;
-                __builtin_amdgcn_global_load_lds(
-                    (gptr_t)(Ag + ((uint64_t)(c >> 2) * nsub + 2 * s) * WIDE_SUB + (c & 3) * 1024 + l16),
-                    (lptr_t)(buf + c * 1024), 16, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lptr_t)(buf + c * 1024), 16, l16,
+                                                         ((c >> 2) * (uint32_t)nsub + 2 * s) * WIDE_SUB + (c & 3) * 1024, 0, 0);
             }
         };
         WideW<FMT> w[WIDE_NT];
         stage(0, As0);
 #pragma unroll
-        for (int t = 0; t < WIDE_NT; t++) { w[t].hdr(rec[t], n); w[t].half(rec[t], lane, 0); }
+        for (int t = 0; t < WIDE_NT; t++) { w[t].hdr(rsW, rec[t], l16); w[t].half(rsW, rec[t], l16, 0); }
         __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0): the direct loads are in LDS
         __syncthreads();
         const uint32_t ns = (sb1 - sb0) * 4;
         for (uint32_t sb = sb0; sb < sb1; sb++) {
-            const bool more = sb + 1 < sb1;
+            const uint32_t step = sb + 1 < sb1 ? REC : 0;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const uint32_t s = (sb - sb0) * 4 + q;
@@ -270,17 +279,25 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
                                 (lptr_t)(Ss + c * 1024), 16, 0, 0);
                     }
                 }
-                WideW<FMT> wn[WIDE_NT];                 // the next half's quants (and header), in flight during this stage
-                if (q == 1) {
+                if constexpr (MIN) {
+                    if (q == 3) {
+                        // minus dmin * sum_ib m_ib (sum of sub-block ib): the sums, split in three fp16
+                        // parts (K-slots 8p + ib), times the integer mins
 #pragma unroll
-                    for (int t = 0; t < WIDE_NT; t++) { wn[t] = w[t]; wn[t].half(rec[t], lane, 1); }
-                }
-                if (q == 3) {
+                        for (int t = 0; t < WIDE_NT; t++) {
+                            v8h mb8;
 #pragma unroll
-                    for (int t = 0; t < WIDE_NT; t++) {
-                        rec[t] += more ? REC : 0;
-                        wn[t].hdr(rec[t], n);
-                        wn[t].half(rec[t], lane, 0);
+                            for (int ib = 0; ib < 8; ib++) mb8[ib] = (_Float16)(float)kq_m(w[t].h, ib);
+                            const float dm = -32.0f * h2f(w[t].h.x >> 16);
+#pragma unroll
+                            for (int mt = 0; mt < MTL; mt++) {
+                                const v8h sf = *(const v8h *)(Ss + mt * 1024 + l16);
+                                const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_f16(sf, mb8, z4, 0, 0, 0);
+#pragma unroll
+                                for (int i = 0; i < 4; i++) acc[mt][t][i] = fmaf(d[i], dm, acc[mt][t][i]);
+                                asm volatile("" : "+v"(acc[mt][t]));
+                            }
+                        }
                     }
                 }
 #pragma unroll
@@ -294,67 +311,65 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
                         if constexpr (FMT == T_Q6_K) { dl[t] = w[t].scale16(ib, 0); dl2[t] = w[t].scale16(ib, 1); }
                         else dl[t] = w[t].scale(ib);
                     }
+                    // the last decode of a half: its registers take the next half's quants (and header), in
+                    // flight during this sub-block's products
+                    if (sub == 1 && q == 1) {
 #pragma unroll
-                    for (int mt = 0; mt < MTL; mt++) {
-                        const uint8_t *ap = cur + (mt * 2 + sub) * WIDE_SUB + lane * 16;
-                        const v8h ah = *(const v8h *)ap, al = *(const v8h *)(ap + 1024);
-                        v4f d[WIDE_NT];
-                        if constexpr (FMT == T_Q6_K) {
-                            const v4h al0 = { al[0], al[1], al[2], al[3] }, al1 = { al[4], al[5], al[6], al[7] };
-                            const v4h ah0 = { ah[0], ah[1], ah[2], ah[3] }, ah1 = { ah[4], ah[5], ah[6], ah[7] };
-                            v4f e[WIDE_NT];
+                        for (int t = 0; t < WIDE_NT; t++) w[t].half(rsW, rec[t], l16, 1);
+                    }
+                    if (sub == 1 && q == 3) {
 #pragma unroll
-                            for (int t = 0; t < WIDE_NT; t++) {
-                                const v4h b0 = { B[t][0], B[t][1], B[t][2], B[t][3] }, b1 = { B[t][4], B[t][5], B[t][6], B[t][7] };
-                                d[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(al0, b0, z4, 0, 0, 0);
-                                e[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(al1, b1, z4, 0, 0, 0);
-                                d[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah0, b0, d[t], 0, 0, 0);
-                                e[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah1, b1, e[t], 0, 0, 0);
+                        for (int t = 0; t < WIDE_NT; t++) {
+                            rec[t] += step;
+                            w[t].hdr(rsW, rec[t], l16);
+                            w[t].half(rsW, rec[t], l16, 0);
+                        }
+                    }
+                    // products of row tile mt beside the multiply-adds of tile mt - 1 and the operand reads of mt + 1
+                    v8h ah[2], al[2];
+                    v4f d[2][WIDE_NT], e[2][WIDE_NT];
+                    const uint8_t *ap = cur + sub * WIDE_SUB + l16;
+                    al[0] = *(const v8h *)(ap + 1024);
+                    ah[0] = *(const v8h *)ap;
+#pragma unroll
+                    for (int mt = 0; mt <= MTL; mt++) {
+                        const int x = mt & 1, y = x ^ 1;
+                        if (mt + 1 < MTL) {
+                            al[y] = *(const v8h *)(ap + (mt + 1) * 2 * WIDE_SUB + 1024);
+                            ah[y] = *(const v8h *)(ap + (mt + 1) * 2 * WIDE_SUB);
+                        }
+                        if (mt < MTL) {
+                            if constexpr (FMT == T_Q6_K) {
+                                const v4h al0 = { al[x][0], al[x][1], al[x][2], al[x][3] }, al1 = { al[x][4], al[x][5], al[x][6], al[x][7] };
+                                const v4h ah0 = { ah[x][0], ah[x][1], ah[x][2], ah[x][3] }, ah1 = { ah[x][4], ah[x][5], ah[x][6], ah[x][7] };
+#pragma unroll
+                                for (int t = 0; t < WIDE_NT; t++) {
+                                    const v4h b0 = { B[t][0], B[t][1], B[t][2], B[t][3] }, b1 = { B[t][4], B[t][5], B[t][6], B[t][7] };
+                                    d[x][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(al0, b0, z4, 0, 0, 0);
+                                    e[x][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(al1, b1, z4, 0, 0, 0);
+                                    d[x][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah0, b0, d[x][t], 0, 0, 0);
+                                    e[x][t] = __builtin_amdgcn_mfma_f32_16x16x16f16(ah1, b1, e[x][t], 0, 0, 0);
+                                }
+                            } else {
+#pragma unroll
+                                for (int t = 0; t < WIDE_NT; t++) d[x][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[x], B[t], z4, 0, 0, 0);
+#pragma unroll
+                                for (int t = 0; t < WIDE_NT; t++) d[x][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[x], B[t], d[x][t], 0, 0, 0);
                             }
+                        }
+                        if (mt > 0) {
 #pragma unroll
                             for (int t = 0; t < WIDE_NT; t++)
 #pragma unroll
                                 for (int i = 0; i < 4; i++)
-                                    acc[mt][t][i] = fmaf(d[t][i], dl[t], fmaf(e[t][i], dl2[t], acc[mt][t][i]));
-                        } else {
+                                    acc[mt - 1][t][i] = FMT == T_Q6_K
+                                        ? fmaf(d[y][t][i], dl[t], fmaf(e[y][t][i], dl2[t], acc[mt - 1][t][i]))
+                                        : fmaf(d[y][t][i], dl[t], acc[mt - 1][t][i]);
+                            // (they are otherwise moved to the end of the loop body, and the products spilled until then)
 #pragma unroll
-                            for (int t = 0; t < WIDE_NT; t++) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, B[t], z4, 0, 0, 0);
-#pragma unroll
-                            for (int t = 0; t < WIDE_NT; t++) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, B[t], d[t], 0, 0, 0);
-#pragma unroll
-                            for (int t = 0; t < WIDE_NT; t++)
-#pragma unroll
-                                for (int i = 0; i < 4; i++) acc[mt][t][i] = fmaf(d[t][i], dl[t], acc[mt][t][i]);
-                        }
-                        // the multiply-adds stay with their products (they are otherwise moved to the end
-                        // of the loop body, and the products spilled until then)
-#pragma unroll
-                        for (int t = 0; t < WIDE_NT; t++) asm volatile("" : "+v"(acc[mt][t]));
-                    }
-                }
-                if constexpr (MIN) {
-                    if (q == 3) {
-                        // minus dmin * sum_ib m_ib (sum of sub-block ib): the sums, split in three fp16
-                        // parts (K-slots 8p + ib), times the integer mins
-#pragma unroll
-                        for (int t = 0; t < WIDE_NT; t++) {
-                            v8h mb8;
-#pragma unroll
-                            for (int ib = 0; ib < 8; ib++) mb8[ib] = (_Float16)(float)kq_m(w[t].h, ib);
-                            const float dm = -32.0f * h2f(w[t].h.x >> 16);
-#pragma unroll
-                            for (int mt = 0; mt < MTL; mt++) {
-                                const v8h sf = *(const v8h *)(Ss + mt * 1024 + lane * 16);
-                                const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_f16(sf, mb8, z4, 0, 0, 0);
-#pragma unroll
-                                for (int i = 0; i < 4; i++) acc[mt][t][i] = fmaf(d[i], dm, acc[mt][t][i]);
-                            }
+                            for (int t = 0; t < WIDE_NT; t++) asm volatile("" : "+v"(acc[mt - 1][t]));
                         }
                     }
-                }
-                if (q == 1 || q == 3) {
-#pragma unroll
-                    for (int t = 0; t < WIDE_NT; t++) w[t] = wn[t];
                 }
                 __builtin_amdgcn_s_waitcnt(0x0F70);
                 __syncthreads();
@@ -734,8 +749,6 @@ extern "C" int qgpu_wide_gemm(qgpu_wide *w, const qgpu_tensor *const *Ws, int n_
             m.rows = (uint32_t)Ws[j]->ne1;
             m.nt16 = (uint32_t)((Ws[j]->ne1 + 15) / 16);
         }
-        // tokens per block by the tokens of the call: a block's decode work does not shrink with its tokens, so
-        // the smallest tile that holds them all, at most 128
         const bool narrow = type == T_Q6_K || type == T_Q8_0;   // their records take more registers: 64 tokens at most
         const int mtl = n <= 32 ? 2 : (n <= 64 || narrow) ? 4 : 8;
         rc = mtl == 2 ? wide_launch<2>(type, a) : mtl == 4 ? wide_launch<4>(type, a) : wide_launch<8>(type, a);
