@@ -624,7 +624,7 @@ extern "C" int qgpu_wide_create(int max_rows, uint64_t max_k, int n_ctx, int n_k
     w->n_ctx = n_ctx;
     w->n_kv = n_kv;
     if (e == hipSuccess && n_ctx && n_kv) e = hipMalloc((void **)&w->kv, ((size_t)n_ctx + 31) / 32 * n_kv * 65536);
-    w->gdn_heads = n_k + 2 * n_v;
+    w->gdn_heads = n_k + 3 * n_v;
     w->gdn_chan = 2 * n_k + n_v;
     if (e == hipSuccess && n_k && n_v) e = hipMalloc((void **)&w->y, (size_t)w->rows * w->gdn_chan * 128 * sizeof(float));
     if (e == hipSuccess && n_k && n_v) e = hipMalloc((void **)&w->gate, (size_t)w->rows * w->gdn_heads * sizeof(float));

@@ -238,7 +238,7 @@ struct WideGdn {
     const float *dtb, *sa, *sin;
     float *sout;              // states before the first and after the last token
     float *y;                 // [M][channels]: q (normalised, / sqrt(128)), k (normalised), v
-    float *gb, *gd, *gk;      // [head][ldg]: beta and decay per v-head, k.q per k-head
+    float *gb, *gd, *gr, *gk; // [head][ldg]: beta, decay and its reciprocal per v-head, k.q per k-head
     float *out;
     uint64_t ldo;
     uint32_t M, ldg;
@@ -256,13 +256,35 @@ __global__ __launch_bounds__(256) void k_wide_conv(const WideGdn p)
     const int grp = blockIdx.y;
     const uint32_t chan = (uint32_t)(2 * p.n_k + p.n_v) * GW_HK;
     if (grp == p.n_k + p.n_v) {
-        const uint32_t nt = min((blockIdx.x + 1) * 4 * GW_TT, p.M) - blockIdx.x * 4 * GW_TT;
-        for (uint32_t e = threadIdx.x; e < nt * p.n_v; e += 256) {
-            const uint32_t t = blockIdx.x * 4 * GW_TT + e / p.n_v, h = e % p.n_v;
-            const float b = p.beta[t * p.ldba + h], av = p.alpha[t * p.ldba + h] + p.dtb[h];
-            const float sp = av > 30.0f ? av : log1pf(expf(av));
-            p.gb[(uint64_t)h * p.ldg + t] = 1.0f / (1.0f + expf(-b));
-            p.gd[(uint64_t)h * p.ldg + t] = expf(p.sa[h] * sp);
+        // the gates of a v-head for a group of 8 tokens (tokens past the end, up to the recurrence's step of
+        // 32: a step that changes nothing): the decay since the group's start and its reciprocal, or, where
+        // that product gets too small to divide by, the token's own decay and 0 for the whole group
+        for (uint32_t e = threadIdx.x; e < 4u * p.n_v; e += 256) {
+            const uint32_t tg = blockIdx.x * 4 * GW_TT + (e / p.n_v) * GW_TT, h = e % p.n_v;
+            float dec[GW_TT], all = 1.0f, D = 1.0f;
+#pragma unroll
+            for (int u = 0; u < GW_TT; u++) {
+                const uint32_t t = tg + u;
+                float b = 0.0f;
+                dec[u] = 1.0f;
+                if (t < p.M) {
+                    const float av = p.alpha[t * p.ldba + h] + p.dtb[h];
+                    const float sp = av > 30.0f ? av : log1pf(expf(av));
+                    dec[u] = expf(p.sa[h] * sp);
+                    b = 1.0f / (1.0f + expf(-p.beta[t * p.ldba + h]));
+                } else if (h < (uint32_t)p.n_k) {
+                    p.gk[(uint64_t)h * p.ldg + t] = 0.0f;
+                }
+                p.gb[(uint64_t)h * p.ldg + t] = b;
+                all *= dec[u];
+            }
+            const bool one = all > 0x1p-40f && all < 0x1p40f;
+#pragma unroll
+            for (int u = 0; u < GW_TT; u++) {
+                D *= dec[u];
+                p.gd[(uint64_t)h * p.ldg + tg + u] = one ? D : dec[u];
+                p.gr[(uint64_t)h * p.ldg + tg + u] = one ? 1.0f / D : 0.0f;
+            }
         }
         return;
     }
@@ -329,86 +351,140 @@ __global__ __launch_bounds__(256) void k_wide_conv(const WideGdn p)
 }
 
 // The delta rule over all tokens, one launch: state rows are independent, so a wave keeps eight of
-// them in registers (16 lanes x 8 columns for a pair of rows) from the first token to the last.
-// Bound by the chain of M steps: about 85 vector operations a step and wave at one wave per SIMD; two
-// rows per lane halve the q and k a row needs from L1.  q, k, v and the gates of the next four tokens
-// load while four are applied.
-#define GW_U 4
-__global__ __launch_bounds__(256, 1) void k_wide_recur(const WideGdn p)
+// them in registers (8 lanes x 16 columns each) from the first token to the last.  Bound by the
+// instructions of the chain of M steps at one wave per SIMD (about 95 a step), once the loads are far
+// enough ahead: y is larger than an L2, so its latency is over a microsecond, eight steps or more.  q, k,
+// v and the gates go to LDS by direct loads, one instruction per token for q and k, four groups of eight
+// tokens deep.  The decay is applied once per group: within one the registers hold S / D, D the decay
+// since the group's start, so a step is one multiply-add per element.
+// Measured at 48 heads, 1992 tokens: 691 us with loads to registers four tokens ahead and the decay in
+// every step, 478 us with the LDS ring, 427 us so (464 us with 16 lanes x 8 columns for a pair of rows:
+// half the LDS reads, more reduction steps).
+// A wave per block spreads the n_v * 16 waves over all compute units; the waves of a head share an
+// XCD's L2 where the heads divide the XCDs.
+#define GW_U 8                            // tokens per group
+#define GW_V    (GW_U * 1024)             // a group in LDS: q and k of each token, then v (8 rows),
+#define GW_G    (GW_V + GW_U * 32)        // then the gates (beta, decay, 1 / decay, k.q)
+#define GW_RING (GW_G + 256)
+__global__ __launch_bounds__(64, 1) void k_wide_recur(const WideGdn p)
 {
-    const int lane = threadIdx.x & 63, cc = lane & 15;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int h = blockIdx.x >> 2, kh = h % p.n_k;
-    const int j = (blockIdx.x & 3) * 32 + wv * 8 + (lane >> 4) * 2;          // rows j, j + 1
-    const uint32_t chan = (uint32_t)(2 * p.n_k + p.n_v) * GW_HK;
-    const uint64_t so = ((uint64_t)h * GW_HK + j) * GW_HK + cc * 4;
-    float S[2][8];
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const float4 v = *(const float4 *)(p.sin + so + r * GW_HK + i * 64);
-            S[r][4 * i] = v.x; S[r][4 * i + 1] = v.y; S[r][4 * i + 2] = v.z; S[r][4 * i + 3] = v.w;
-        }
-    const float *yq = p.y + kh * GW_HK + cc * 4, *yk = yq + p.n_k * GW_HK;
-    const float *yv = p.y + 2 * p.n_k * GW_HK + h * GW_HK + j;
-    const float *gb = p.gb + (uint64_t)h * p.ldg, *gd = p.gd + (uint64_t)h * p.ldg, *gk = p.gk + (uint64_t)kh * p.ldg;
-    struct Tok { float4 q[2], k[2]; float2 v; float b, d, kq; };
-    Tok cur[GW_U], nxt[GW_U];
-    auto load = [&](Tok *T, uint32_t t) {
-#pragma unroll
-        for (int u = 0; u < GW_U; u++) {
-            const uint32_t tt = min(t + u, p.M - 1);
-            const uint64_t o = (uint64_t)tt * chan;
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                T[u].q[i] = *(const float4 *)(yq + o + i * 64);
-                T[u].k[i] = *(const float4 *)(yk + o + i * 64);
-            }
-            T[u].v = *(const float2 *)(yv + o);
-            T[u].b = gb[tt];
-            T[u].d = gd[tt];
-            T[u].kq = gk[tt];
-        }
-    };
-    load(cur, 0);
-    for (uint32_t t0 = 0; t0 < p.M; t0 += GW_U) {
-        load(nxt, t0 + GW_U);
-#pragma unroll
-        for (int u = 0; u < GW_U; u++) {
-            if (t0 + u >= p.M) break;
-            const float q[8] = { cur[u].q[0].x, cur[u].q[0].y, cur[u].q[0].z, cur[u].q[0].w,
-                                 cur[u].q[1].x, cur[u].q[1].y, cur[u].q[1].z, cur[u].q[1].w };
-            const float k[8] = { cur[u].k[0].x, cur[u].k[0].y, cur[u].k[0].z, cur[u].k[0].w,
-                                 cur[u].k[1].x, cur[u].k[1].y, cur[u].k[1].z, cur[u].k[1].w };
-            float o[2];
-#pragma unroll
-            for (int r = 0; r < 2; r++) {
-                float sk0 = 0.0f, sq0 = 0.0f, sk1 = 0.0f, sq1 = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    sk0 = fmaf(S[r][i], k[i], sk0);
-                    sk1 = fmaf(S[r][4 + i], k[4 + i], sk1);
-                    sq0 = fmaf(S[r][i], q[i], sq0);
-                    sq1 = fmaf(S[r][4 + i], q[4 + i], sq1);
-                }
-                const float sk = rowsum16(sk0 + sk1), sq = rowsum16(sq0 + sq1);
-                const float vj = r ? cur[u].v.y : cur[u].v.x;
-                const float dj = (vj - cur[u].d * sk) * cur[u].b;
-                o[r] = fmaf(dj, cur[u].kq, cur[u].d * sq);
-#pragma unroll
-                for (int i = 0; i < 8; i++) S[r][i] = fmaf(dj, k[i], cur[u].d * S[r][i]);
-            }
-            if (cc == 0) *(float2 *)(p.out + (uint64_t)(t0 + u) * p.ldo + (uint64_t)h * GW_HK + j) = make_float2(o[0], o[1]);
-        }
-#pragma unroll
-        for (int u = 0; u < GW_U; u++) cur[u] = nxt[u];
+    __shared__ __attribute__((aligned(16))) uint8_t R0[GW_RING], R1[GW_RING], R2[GW_RING], R3[GW_RING];
+    const int lane = threadIdx.x & 63, cc = lane & 7;
+    int h = blockIdx.x >> 4, part = blockIdx.x & 15;
+    if (p.n_v % 8 == 0) {
+        const int i = blockIdx.x >> 3;
+        h = (i >> 4) * 8 + (blockIdx.x & 7);
+        part = i & 15;
     }
+    const int kh = h % p.n_k, j = part * 8 + (lane >> 3);
+    const uint32_t chan4 = (uint32_t)(2 * p.n_k + p.n_v) * GW_HK * 4, last = p.M - 1;
+    const uint64_t so = ((uint64_t)h * GW_HK + j) * GW_HK + cc * 4;
+    float S[16];
 #pragma unroll
-    for (int r = 0; r < 2; r++)
+    for (int i = 0; i < 4; i++) {
+        const float4 v = *(const float4 *)(p.sin + so + i * 32);
+        S[4 * i] = v.x; S[4 * i + 1] = v.y; S[4 * i + 2] = v.z; S[4 * i + 3] = v.w;
+    }
+    const __amdgpu_buffer_rsrc_t rsK = __builtin_amdgcn_make_buffer_rsrc((void *)(p.y + kh * GW_HK), 0, 0x7FFFFFFF, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsV = __builtin_amdgcn_make_buffer_rsrc((void *)(p.y + (2 * p.n_k + h) * GW_HK + part * 8), 0, 0x7FFFFFFF, 0x00020000);
+    const uint32_t oqk = lane < 32 ? (uint32_t)lane * 16 : (uint32_t)(p.n_k * GW_HK * 4 + (lane - 32) * 16);
+    const __amdgpu_buffer_rsrc_t rsG = __builtin_amdgcn_make_buffer_rsrc((void *)p.gb, 0, 0x7FFFFFFF, 0x00020000);
+    const uint32_t grow = (lane & 3) * p.n_v + ((lane & 3) == 3 ? kh : h);     // beta, decay, reciprocal, k.q rows
+    // tokens past the end load the last one's rows (and gates that leave the state as it is)
+    auto load = [&](uint8_t *R, uint32_t t) {
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-            *(float4 *)(p.sout + so + r * GW_HK + i * 64) = make_float4(S[r][4 * i], S[r][4 * i + 1], S[r][4 * i + 2], S[r][4 * i + 3]);
+        for (int u = 0; u < GW_U; u++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsK, (lptr_t)(R + u * 1024), 16, oqk, min(t + u, last) * chan4, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsV, (lptr_t)(R + GW_V), 4,
+                                                 min(t + (lane >> 3), last) * chan4 + (lane & 7) * 4, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsG, (lptr_t)(R + GW_G), 4,
+                                                 lane < 4 * GW_U ? (grow * p.ldg + min(t + (lane >> 2), p.ldg - 1)) * 4 : 0x80000000u,
+                                                 0, 0, 0);
+    };
+    // lane cc of a row keeps the group's token cc: one store per group (tokens past the end have an offset
+    // past the buffer)
+    const __amdgpu_buffer_rsrc_t rsO = __builtin_amdgcn_make_buffer_rsrc((void *)(p.out + (uint64_t)h * GW_HK), 0, 0x7FFFFFFF, 0x00020000);
+    const uint32_t ldo4 = (uint32_t)p.ldo * 4, oo = (uint32_t)cc * ldo4 + (uint32_t)j * 4;
+    struct Tok { float4 q[4], k[4], gt; float v; };
+    auto read = [&](const uint8_t *R, int u) {
+        Tok T;
+        const uint8_t *r = R + u * 1024 + cc * 16;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            T.k[i] = *(const float4 *)(r + 512 + i * 128);
+            T.q[i] = *(const float4 *)(r + i * 128);
+        }
+        T.v = *(const float *)(R + GW_V + u * 32 + (lane >> 3) * 4);
+        T.gt = *(const float4 *)(R + GW_G + u * 16);
+        return T;
+    };
+    // one token: the registers hold S / D before and after (rD = 1 / D); its output
+    auto token = [&](const Tok &T, float D, float rD) {
+        float q[16], k[16], sk[4], sq[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            q[4 * i] = T.q[i].x; q[4 * i + 1] = T.q[i].y; q[4 * i + 2] = T.q[i].z; q[4 * i + 3] = T.q[i].w;
+            k[4 * i] = T.k[i].x; k[4 * i + 1] = T.k[i].y; k[4 * i + 2] = T.k[i].z; k[4 * i + 3] = T.k[i].w;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) { sk[i] = S[i] * k[i]; sq[i] = S[i] * q[i]; }
+#pragma unroll
+        for (int i = 4; i < 16; i++) {
+            sk[i & 3] = fmaf(S[i], k[i], sk[i & 3]);
+            sq[i & 3] = fmaf(S[i], q[i], sq[i & 3]);
+        }
+        float a = (sk[0] + sk[1]) + (sk[2] + sk[3]), b = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+        a += dpp_mov<0xB1>(a);  b += dpp_mov<0xB1>(b);           // the row's eight lanes
+        a += dpp_mov<0x4E>(a);  b += dpp_mov<0x4E>(b);
+        a += dpp_mov<0x141>(a); b += dpp_mov<0x141>(b);
+        const float d = fmaf(-D, a, T.v) * T.gt.x, c = d * rD;
+#pragma unroll
+        for (int i = 0; i < 16; i++) S[i] = fmaf(c, k[i], S[i]);
+        return fmaf(d, T.gt.w, D * b);
+    };
+    auto apply = [&](const uint8_t *R, uint32_t t) {
+        float out = 0.0f;
+        if (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, *(const float *)(R + GW_G + 8)))) {
+            Tok T[2];
+            T[0] = read(R, 0);
+#pragma unroll
+            for (int u = 0; u < GW_U; u++) {
+                if (u + 1 < GW_U) T[(u + 1) & 1] = read(R, u + 1);
+                const Tok &x = T[u & 1];
+                const float o = token(x, x.gt.y, x.gt.z);
+                out = cc == u ? o : out;
+                if (u + 1 == GW_U)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) S[i] *= x.gt.y;
+            }
+        } else {                                             // the decay token by token
+#pragma unroll 1
+            for (int u = 0; u < GW_U; u++) {
+                const Tok x = read(R, u);
+#pragma unroll
+                for (int i = 0; i < 16; i++) S[i] *= x.gt.y;
+                const float o = token(x, 1.0f, 1.0f);
+                out = cc == u ? o : out;
+            }
+        }
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, out), rsO, t + cc < p.M ? oo : 0x80000000u, t * ldo4, 0);
+    };
+    // a group is in LDS when at most the three groups issued after it (ten loads each) are in flight
+#define GW_STEP(RL, RA, T) do { load(RL, (T) + 3 * GW_U); asm volatile("s_waitcnt vmcnt(30)" ::: "memory"); apply(RA, T); } while (0)
+    load(R0, 0);
+    load(R1, GW_U);
+    load(R2, 2 * GW_U);
+    for (uint32_t t = 0; t < p.M; t += 4 * GW_U) {
+        GW_STEP(R3, R0, t);
+        GW_STEP(R0, R1, t + GW_U);
+        GW_STEP(R1, R2, t + 2 * GW_U);
+        GW_STEP(R2, R3, t + 3 * GW_U);
+    }
+#undef GW_STEP
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // no direct load may land after the block's LDS is given back
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        *(float4 *)(p.sout + so + i * 32) = make_float4(S[4 * i], S[4 * i + 1], S[4 * i + 2], S[4 * i + 3]);
 }
 
 extern "C" int qgpu_wide_gdn(qgpu_wide *w, const float *x, uint64_t ldx, int n, const float *conv_w,
@@ -420,19 +496,20 @@ extern "C" int qgpu_wide_gdn(qgpu_wide *w, const float *x, uint64_t ldx, int n, 
     if (rc) return rc;
     if (head_dim != GW_HK) return QGPU_E_RANGE;
     if (!w || !x || !conv_w || !conv_in || !conv_out || !beta_raw || !alpha_raw || !dt_bias || !ssm_a || !ssm_in ||
-        !ssm_out || !out || n < 1 || n > w->rows || n_k < 1 || n_v < 1 || n_v % n_k || n_k + 2 * n_v > w->gdn_heads ||
-        (2 * n_k + n_v) > w->gdn_chan || ldx % 2 || ldo % 2 || !al16(x) || !al16(conv_w) || !al16(conv_in) ||
+        !ssm_out || !out || n < 1 || n > w->rows || n_k < 1 || n_v < 1 || n_v % n_k || n_k + 3 * n_v > w->gdn_heads ||
+        (2 * n_k + n_v) > w->gdn_chan || ldx % 2 || ldo % 2 || (uint64_t)n * ldo >= (1u << 29) || (uint64_t)n * w->gdn_chan >= (1u << 22) || !al16(x) || !al16(conv_w) || !al16(conv_in) ||
         !al16(conv_out) || !al16(ssm_in) || !al16(ssm_out) || !al16(out))
         return QGPU_E_ARG;
     WideGdn p = {};
     p.x = x; p.ldx = ldx; p.cw = conv_w; p.cin = conv_in; p.cout = conv_out; p.beta = beta_raw; p.alpha = alpha_raw;
     p.ldba = ldba; p.dtb = dt_bias; p.sa = ssm_a; p.sin = ssm_in; p.sout = ssm_out; p.y = w->y;
     p.ldg = (uint32_t)w->rows;
-    p.gb = w->gate; p.gd = p.gb + (uint64_t)n_v * p.ldg; p.gk = p.gd + (uint64_t)n_v * p.ldg;
+    p.gb = w->gate; p.gd = p.gb + (uint64_t)n_v * p.ldg; p.gr = p.gd + (uint64_t)n_v * p.ldg;
+    p.gk = p.gr + (uint64_t)n_v * p.ldg;
     p.out = out; p.ldo = ldo; p.M = (uint32_t)n; p.n_k = n_k; p.n_v = n_v; p.eps = eps;
     hipLaunchKernelGGL(k_wide_conv, dim3((n + 4 * GW_TT - 1) / (4 * GW_TT), n_k + n_v + 1), dim3(256), 0, qg::stream, p);
     QG_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_wide_recur, dim3(n_v * 4), dim3(256), 0, qg::stream, p);
+    hipLaunchKernelGGL(k_wide_recur, dim3(n_v * 16), dim3(64), 0, qg::stream, p);
     QG_LAUNCH_CHECK();
     return QGPU_OK;
 }

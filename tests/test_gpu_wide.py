@@ -190,14 +190,16 @@ def test_wide_attention_head_counts(gpu, nh, nkv):
 
 # ---------------------------------------------------------------- Gated DeltaNet
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 8, 33, 100])
-@pytest.mark.parametrize("nk,nv", [(16, 48), (2, 4)])
-def test_wide_gdn_vs_batches(gpu, n, nk, nv):
-    """against the same tokens in batches of 8 (qgpu_gdn_fused), which carries its own oracle tests"""
+@pytest.mark.parametrize("nk,nv,gate", [(16, 48, 1.0), (2, 4, 1.0), (2, 4, 40.0)])
+def test_wide_gdn_vs_batches(gpu, n, nk, nv, gate):
+    """against the same tokens in batches of 8 (qgpu_gdn_fused), which carries its own oracle tests; with
+    strong gates the decay of a group of 8 tokens leaves fp32 (some single ones too)"""
     hk, eps, slots = 128, 1e-6, 9
     rng = np.random.default_rng(n + nk)
     chan = (2 * nk + nv) * hk
     x = rng.standard_normal((n, chan)).astype(np.float32)
     be, al = (rng.standard_normal((n, nv)).astype(np.float32) for _ in range(2))
+    al *= np.float32(gate)
     cw = (0.5 * rng.standard_normal((chan, 4))).astype(np.float32)
     dtb = (0.5 * rng.standard_normal(nv)).astype(np.float32)
     a = (-(0.3 + 0.7 * np.abs(rng.standard_normal(nv)))).astype(np.float32)
