@@ -189,16 +189,19 @@ int  qgpu_gemv_rows_batch(const qgpu_tensor *W, const float *x, uint64_t ldx, in
  * qgpu_wide_prepare converts act's rows (QGPU_ACT_* without pending planes, gather or xout; a
  * gated norm has heads of 128; x, y, w, w2 16-byte aligned, ldx and ldy multiples of 4) and
  * qgpu_wide_gemm multiplies them, out[t*ldo + r] (+)= sum_i W[r,i] v[t][i], with every matrix of
- * the call (matrix-core formats only: qgpu_wide_supports).  n <= max_rows, ne0 <= max_k.
+ * the call (matrix-core formats only: qgpu_wide_supports).  n <= max_rows, ne0 <= max_k.  sums:
+ * also the sub-block sums that Q4_K and Q5_K matrices multiply their mins with.
+ * qgpu_wide_gemm_silu: out = silu(gate v) * (up v), two matrices of one format and size.
  * n_ctx positions of n_kv heads and n_k / n_v GDN heads size the workspaces of qgpu_wide_attn and
  * qgpu_wide_gdn (0: those calls are rejected). */
 typedef struct qgpu_wide qgpu_wide;
 int  qgpu_wide_create(int max_rows, uint64_t max_k, int n_ctx, int n_kv, int n_k, int n_v, qgpu_wide **out);
 int  qgpu_wide_free(qgpu_wide *w);
 int  qgpu_wide_supports(const qgpu_tensor *W);
-int  qgpu_wide_prepare(qgpu_wide *w, const qgpu_act *act, int n, uint64_t ne0);
+int  qgpu_wide_prepare(qgpu_wide *w, const qgpu_act *act, int n, uint64_t ne0, int sums);
 int  qgpu_wide_gemm(qgpu_wide *w, const qgpu_tensor *const *Ws, int n_mat, int n, float *const *outs,
                     const uint64_t *ldos, int flags);
+int  qgpu_wide_gemm_silu(qgpu_wide *w, const qgpu_tensor *gate, const qgpu_tensor *up, int n, float *out, uint64_t ldo);
 /* qgpu_attn_decode for n tokens at positions pos..pos+n-1 (q prepared and the caches written by
  * qgpu_attn_prep); pos + n <= n_ctx, n_kv as created. */
 int  qgpu_wide_attn(qgpu_wide *w, const float *q, uint64_t ldq, const float *kcache, const float *vcache,

@@ -12,16 +12,19 @@
 // quants) are exact in fp16, every product is exact in fp32, and a sub-block's sum meets its scale
 // (d x the sub-block's integer scale, fp32) in one fp32 multiply-add per output.
 //
-// Layout.  Activations: per (16-row tile, 32-column sub-block) 2 KB, the hi plane then the lo
-// plane, each in the A-operand order of v_mfma_f32_16x16x32_f16: lane g*16 + m holds row m's
-// elements 4g..4g+3 and 16+4g..16+4g+3, the order in which the packed weight records hold
-// their lanes' dwords (gemv.hip), so a lane's nibble dword decodes straight into its B operand.
+// Layout.  Activations: per (16-row tile, 32-column sub-block) 2 KB, one 128-byte line per row: its
+// hi parts, then its lo parts, each in four 16-byte groups g of the elements 4g..4g+3 and
+// 16+4g..16+4g+3.  Group g of row m is lane g*16 + m's A operand of v_mfma_f32_16x16x32_f16, and its
+// order the one in which the packed weight records hold their lanes' dwords (gemv.hip), so a lane's
+// nibble dword decodes straight into its B operand.  The direct loads to LDS put the groups in lane order.
 //
 // Schedule.  A block of 4 waves owns 16*MTL tokens x 256 weight rows (64 per wave: the
 // wave decodes its own weights in registers, and the activation tile is shared through LDS).  The
 // (tile, super-block) units of a launch are cut into equal contiguous runs, one per resident
 // block; a tile that more than one block computes leaves partial sums that k_wide_fix adds in
-// block order, so results do not depend on timing.
+// block order, so results do not depend on timing.  (Adding them in the block that counts in last
+// instead was no faster with two blocks per tile and 1.9x slower with seven: 17408 -> 5120 at 512
+// tokens 199 -> 376 us, one block reading what the fix kernel spreads over all units.)
 #include "qgpu_internal.h"
 #include <new>
 
@@ -29,6 +32,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
 #define WIDE_NT    4                    // 16-row weight tiles per wave
 #define WIDE_N     (4 * WIDE_NT * 16)   // weight rows per block
@@ -43,14 +47,21 @@ struct WideMat {
 };
 struct WideArgs {
     WideMat m[QGPU_MAX_MULTI];
-    int n_mat, accum;
+    int n_mat, accum, pair;             // pair: m[0] and m[1] are a gate and its up projection (WIDE_PAIR)
     uint32_t nsb, M, mblk, G, U;        // super-blocks, tokens, token blocks, blocks, units
     const uint8_t *A, *S;
     const float *xs;
     float *piece;
 };
 
+// block that computes unit u
+static __host__ __device__ __forceinline__ uint32_t unit_block(uint32_t u, uint32_t G, uint32_t U)
+{
+    return (uint32_t)((((uint64_t)u + 1) * G - 1) / U);
+}
+
 static __device__ __forceinline__ float h2f(uint32_t h16) { return (float)__builtin_bit_cast(_Float16, (unsigned short)h16); }
+static __device__ __forceinline__ float silu_w(float v) { return v / (1.0f + expf(-v)); }
 static __device__ __forceinline__ uint32_t u4_get(uint4 v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
 // four unsigned bytes u -> four fp16 values u - 128 (0x6400 | u is 1024 + u; the sum is exact), two per dword
@@ -226,39 +237,46 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
     const uint32_t ue = (uint32_t)((uint64_t)(g + 1) * a.U / a.G);
     const uint64_t nsub = (uint64_t)a.nsb * 8;
     const uint32_t l16 = (uint32_t)lane * 16;
+    // lane g*16 + m fetches part g of row m: rows lie in memory one after the other, operands lane by lane in LDS
+    const uint32_t va = (uint32_t)n * 128 + (uint32_t)(lane >> 4) * 16, vs = (uint32_t)n * 64 + (uint32_t)(lane >> 4) * 16;
     const v4f z4 = { 0.0f, 0.0f, 0.0f, 0.0f };
     while (u < ue) {
         const uint32_t tile = u / a.nsb, sb0 = u - tile * a.nsb, sb1 = min(a.nsb, sb0 + (ue - u));
         const uint32_t nt = tile / a.mblk, mb = tile - nt * a.mblk;
         int j = 0;
-        while (j + 1 < a.n_mat && nt >= a.m[j + 1].tile0) j++;
-        const uint32_t row0 = (nt - a.m[j].tile0) * WIDE_N + wv * (WIDE_NT * 16);   // this wave's first weight row
+        while (!a.pair && j + 1 < a.n_mat && nt >= a.m[j + 1].tile0) j++;
+        // this wave's first weight row; a pair's block holds 128 rows of each matrix, tiles 0, 1 of a wave the gate's
+        const uint32_t row0 = (nt - a.m[j].tile0) * (a.pair ? WIDE_N / 2 : WIDE_N) + wv * (a.pair ? WIDE_NT * 8 : WIDE_NT * 16);
         // its records: past the matrix's end any loadable one (the results are dropped)
         const uint32_t tstr = a.nsb * REC, t0 = min(row0 / 16, a.m[j].nt16 - 1);
         const rsrc_t rsW = __builtin_amdgcn_make_buffer_rsrc((void *)(a.m[j].W + (uint64_t)t0 * tstr), 0, 0x7FFFFFFF, 0x00020000);
+        const rsrc_t rsU = __builtin_amdgcn_make_buffer_rsrc((void *)((a.pair ? a.m[1].W : a.m[j].W) + (uint64_t)t0 * tstr), 0, 0x7FFFFFFF, 0x00020000);
         uint32_t rec[WIDE_NT];
 #pragma unroll
-        for (int t = 0; t < WIDE_NT; t++) rec[t] = min((uint32_t)t, a.m[j].nt16 - 1 - t0) * tstr + sb0 * REC;
+        for (int t = 0; t < WIDE_NT; t++)
+            rec[t] = min((uint32_t)(a.pair ? t % (WIDE_NT / 2) : t), a.m[j].nt16 - 1 - t0) * tstr + sb0 * REC;
+#define RSW(t) ((t) < WIDE_NT / 2 ? rsW : rsU)
         v4f acc[MTL][WIDE_NT];
 #pragma unroll
         for (int mt = 0; mt < MTL; mt++)
 #pragma unroll
             for (int t = 0; t < WIDE_NT; t++) acc[mt][t] = z4;
-        // this wave's MTL 1 KB chunks of a stage: chunk c = (row tile c / 4, 1 KB part c % 4)
+        // this wave's MTL 1 KB chunks of a stage: chunk c = (row tile c / 4, sub-block c % 4 / 2, plane c % 2)
         const rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(a.A + ((uint64_t)mb * MTL * nsub + (uint64_t)sb0 * 8) * WIDE_SUB), 0, 0x7FFFFFFF, 0x00020000);
         auto stage = [&](uint32_t s, uint8_t *buf) {
 #pragma unroll
             for (int i = 0; i < MTL; i++) {
                 const int c = wv * MTL + i;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lptr_t)(buf + c * 1024), 16, l16,
-                                                         ((c >> 2) * (uint32_t)nsub + 2 * s) * WIDE_SUB + (c & 3) * 1024, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rsA, (lptr_t)(buf + c * 1024), 16, va,
+                    ((c >> 2) * (uint32_t)nsub + 2 * s) * WIDE_SUB + ((c >> 1) & 1) * WIDE_SUB + (c & 1) * 64, 0, 0);
             }
         };
         WideW<FMT> w[WIDE_NT];
         stage(0, As0);
 #pragma unroll
-        for (int t = 0; t < WIDE_NT; t++) { w[t].hdr(rsW, rec[t], l16); w[t].half(rsW, rec[t], l16, 0); }
+        for (int t = 0; t < WIDE_NT; t++) { w[t].hdr(RSW(t), rec[t], l16); w[t].half(RSW(t), rec[t], l16, 0); }
         __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0): the direct loads are in LDS
         __syncthreads();
         const uint32_t ns = (sb1 - sb0) * 4;
@@ -275,7 +293,7 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
                         const int c = wv + 4 * i;
                         if (c < MTL)
                             __builtin_amdgcn_global_load_lds(
-                                (gptr_t)(a.S + (((uint64_t)mb * MTL + c) * a.nsb + sb) * 1024 + l16),
+                                (gptr_t)(a.S + (((uint64_t)mb * MTL + c) * a.nsb + sb) * 1024 + vs),
                                 (lptr_t)(Ss + c * 1024), 16, 0, 0);
                     }
                 }
@@ -315,14 +333,14 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
                     // flight during this sub-block's products
                     if (sub == 1 && q == 1) {
 #pragma unroll
-                        for (int t = 0; t < WIDE_NT; t++) w[t].half(rsW, rec[t], l16, 1);
+                        for (int t = 0; t < WIDE_NT; t++) w[t].half(RSW(t), rec[t], l16, 1);
                     }
                     if (sub == 1 && q == 3) {
 #pragma unroll
                         for (int t = 0; t < WIDE_NT; t++) {
                             rec[t] += step;
-                            w[t].hdr(rsW, rec[t], l16);
-                            w[t].half(rsW, rec[t], l16, 0);
+                            w[t].hdr(RSW(t), rec[t], l16);
+                            w[t].half(RSW(t), rec[t], l16, 0);
                         }
                     }
                     // products of row tile mt beside the multiply-adds of tile mt - 1 and the operand reads of mt + 1
@@ -375,75 +393,111 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
                 __syncthreads();
             }
         }
+        // ---- a tile shared between blocks: partial sums, in register order, for k_wide_fix
+        if (sb1 - sb0 != a.nsb) {
+            constexpr uint32_t PB = MTL * 16 * WIDE_N * 4;                       // bytes of a piece
+            const uint32_t pv = threadIdx.x * 16;
+            {
+                const rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((char *)a.piece + (uint64_t)(2 * g + (sb0 == 0)) * PB, 0, PB, 0x00020000);
+#pragma unroll
+                for (int mt = 0; mt < MTL; mt++)
+#pragma unroll
+                    for (int t = 0; t < WIDE_NT; t++)
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, acc[mt][t]), rs, pv, (mt * WIDE_NT + t) * 4096, 0);
+            }
+            u += sb1 - sb0;
+            continue;
+        }
         // ---- results: lane (g, n), register i: token 16 mt + 4 g + i, weight row 16 t + n
         const uint32_t g4 = 4 * (uint32_t)(lane >> 4);
-        if (sb0 == 0 && sb1 == a.nsb) {
 #pragma unroll
-            for (int mt = 0; mt < MTL; mt++) {
-                const uint32_t r0 = (mb * MTL + mt) * 16 + g4;
-                const float4 x4 = *(const float4 *)(a.xs + r0);
-                const float xr[4] = { x4.x, x4.y, x4.z, x4.w };
+        for (int mt = 0; mt < MTL; mt++) {
+            const uint32_t r0 = (mb * MTL + mt) * 16 + g4;
+            const float4 x4 = *(const float4 *)(a.xs + r0);
+            const float xr[4] = { x4.x, x4.y, x4.z, x4.w };
+            if (a.pair) {                                    // silu(gate) * up: tiles t and t + 2
 #pragma unroll
-                for (int t = 0; t < WIDE_NT; t++) {
+                for (int t = 0; t < WIDE_NT / 2; t++) {
                     const uint32_t c = row0 + 16 * t + n;
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        if (r0 + i < a.M && c < a.m[j].rows) {
-                            float *o = a.m[j].out + (uint64_t)(r0 + i) * a.m[j].ldo + c;
-                            const float v = acc[mt][t][i] * xr[i];
-                            *o = a.accum ? *o + v : v;
-                        }
+                        if (r0 + i < a.M && c < a.m[0].rows)
+                            a.m[0].out[(uint64_t)(r0 + i) * a.m[0].ldo + c] =
+                                silu_w(acc[mt][t][i] * xr[i]) * (acc[mt][t + WIDE_NT / 2][i] * xr[i]);
                 }
+                continue;
             }
-        } else {
-            float *P = a.piece + (uint64_t)(2 * g + (sb0 == 0)) * (MTL * 16 * WIDE_N) + wv * (WIDE_NT * 16) + n;
 #pragma unroll
-            for (int mt = 0; mt < MTL; mt++)
+            for (int t = 0; t < WIDE_NT; t++) {
+                const uint32_t c = row0 + 16 * t + n;
 #pragma unroll
-                for (int t = 0; t < WIDE_NT; t++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) P[(uint64_t)(mt * 16 + g4 + i) * WIDE_N + 16 * t] = acc[mt][t][i];
+                for (int i = 0; i < 4; i++)
+                    if (r0 + i < a.M && c < a.m[j].rows) {
+                        float *o = a.m[j].out + (uint64_t)(r0 + i) * a.m[j].ldo + c;
+                        const float v = acc[mt][t][i] * xr[i];
+                        *o = a.accum ? *o + v : v;
+                    }
+            }
         }
         u += sb1 - sb0;
     }
 }
 
-// block that computes unit u
-static __host__ __device__ __forceinline__ uint32_t unit_block(uint32_t u, uint32_t G, uint32_t U)
-{
-    return (uint32_t)((((uint64_t)u + 1) * G - 1) / U);
-}
-
-// Adds the pieces of the tiles that several blocks computed, in block order.  Block (tile, quarter of
-// its rows); a block's last piece starts at its tile's first unit (slot 1), its first one does not (slot 0).
+// Adds the pieces of the tiles that several blocks computed, in block order: block (tile, row tile mt),
+// the product kernel's lanes and registers, so pieces are written and read in whole lines, four at a time
+// (17408 -> 5120 at 128 tokens, product and sums, 117 -> 70 us; at 512 199 -> 194 us).  A block's last piece starts at its tile's first unit (slot 1),
+// its first one does not (slot 0).
 template <int MTL>
 __global__ __launch_bounds__(256) void k_wide_fix(const WideArgs a)
 {
-    const uint32_t tile = blockIdx.x, u0 = tile * a.nsb;
+    const uint32_t tile = blockIdx.x, mt = blockIdx.y, u0 = tile * a.nsb;
     const uint32_t ga = unit_block(u0, a.G, a.U), gb = unit_block(u0 + a.nsb - 1, a.G, a.U);
     if (ga == gb) return;
-    const uint32_t nt = tile / a.mblk, mb = tile - nt * a.mblk;
+    const uint32_t nt = tile / a.mblk, mb = tile - nt * a.mblk, wv = threadIdx.x >> 6, n = threadIdx.x & 15;
+    const uint32_t r0 = (mb * MTL + mt) * 16 + 4 * ((threadIdx.x >> 4) & 3);
+    if ((mb * MTL + mt) * 16 >= a.M) return;
+    constexpr uint64_t PS = MTL * 16 * WIDE_N;
+    const float *P = a.piece + mt * WIDE_NT * 1024 + threadIdx.x * 4;
+    v4f s[WIDE_NT];
+#pragma unroll
+    for (int t = 0; t < WIDE_NT; t++) s[t] = *(const v4f *)(P + (uint64_t)(2 * ga + 1) * PS + t * 1024);
+    for (uint32_t q = ga + 1; q <= gb; q += 4) {
+        v4f v[4][WIDE_NT];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int t = 0; t < WIDE_NT; t++) v[k][t] = *(const v4f *)(P + (uint64_t)(2 * min(q + k, gb)) * PS + t * 1024);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int t = 0; t < WIDE_NT; t++)
+                if (q + k <= gb) s[t] += v[k][t];
+    }
+    const float4 x4 = *(const float4 *)(a.xs + r0);
+    const float xr[4] = { x4.x, x4.y, x4.z, x4.w };
+    if (a.pair) {
+#pragma unroll
+        for (int t = 0; t < WIDE_NT / 2; t++) {
+            const uint32_t c = nt * (WIDE_N / 2) + wv * (WIDE_NT * 8) + 16 * t + n;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (r0 + i < a.M && c < a.m[0].rows)
+                    a.m[0].out[(uint64_t)(r0 + i) * a.m[0].ldo + c] = silu_w(s[t][i] * xr[i]) * (s[t + WIDE_NT / 2][i] * xr[i]);
+        }
+        return;
+    }
     int j = 0;
     while (j + 1 < a.n_mat && nt >= a.m[j + 1].tile0) j++;
-    const uint32_t c = (threadIdx.x & 63) * 4, col = (nt - a.m[j].tile0) * WIDE_N + c, rows = a.m[j].rows;
-    constexpr uint64_t PS = MTL * 16 * WIDE_N;
-    if (col >= rows) return;
 #pragma unroll
-    for (int k = 0; k < MTL; k++) {
-        const uint32_t r = blockIdx.y * (MTL * 4) + 4 * k + (threadIdx.x >> 6), row = mb * MTL * 16 + r;
-        if (row >= a.M) break;
-        const float *P = a.piece + (uint64_t)r * WIDE_N + c;
-        float4 s = *(const float4 *)(P + (uint64_t)(2 * ga + 1) * PS);
-        for (uint32_t g = ga + 1; g <= gb; g++) {
-            const float4 v = *(const float4 *)(P + (uint64_t)(2 * g) * PS);
-            s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-        }
-        const float x = a.xs[row];
-        float *o = a.m[j].out + (uint64_t)row * a.m[j].ldo + col;
-        const float v[4] = { s.x * x, s.y * x, s.z * x, s.w * x };
+    for (int t = 0; t < WIDE_NT; t++) {
+        const uint32_t c = (nt - a.m[j].tile0) * WIDE_N + wv * (WIDE_NT * 16) + 16 * t + n;
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            if (col + i < rows) o[i] = a.accum ? o[i] + v[i] : v[i];
+            if (r0 + i < a.M && c < a.m[j].rows) {
+                float *o = a.m[j].out + (uint64_t)(r0 + i) * a.m[j].ldo + c;
+                const float v = s[t][i] * xr[i];
+                *o = a.accum ? *o + v : v;
+            }
     }
 }
 
@@ -453,24 +507,22 @@ struct WidePrep {
     uint64_t ldx, ldy;
     uint32_t M, ne0, seg;               // tokens, columns, segment length (two-segment RMSNorm)
     float eps;
-    uint8_t *A, *S;
+    uint8_t *A, *S;                     // S: NULL when no matrix needs the sums
     float *xs;
 };
 #define WP_CAT 4                        // internal kind: the two-segment RMSNorm
 
-static __device__ __forceinline__ float silu_w(float v) { return v / (1.0f + expf(-v)); }
-
 // One token per block of NTH threads; a thread holds GPT groups of eight elements, each one lane's
 // share of a sub-block (4g..4g+3 and 16+4g..16+4g+3), so the row is read once and the planes
-// are written from registers, 16 bytes per group.  The 16 rows of a tile run on one XCD (block index
-// mod 8), whose L2 collects their 16-byte parts of each 256-byte run.
+// are written from registers: a sub-block's hi and lo parts are one 128-byte line.  Bound by memory
+// traffic in two phases, read then write: 3.4 TB/s at 1992 tokens x 17408 (81 us; 111 us with 256 threads
+// a row and 16-byte parts 256 bytes apart).
 template <int KIND, int GPT, int NTH>
 __global__ __launch_bounds__(NTH) void k_wide_prep(const WidePrep p)
 {
     __shared__ float red[3][NTH / 64];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const uint32_t b = blockIdx.x, r = (((b >> 3) >> 4) * 8 + (b & 7)) * 16 + ((b >> 3) & 15);
-    if (r >= p.M) return;
+    const uint32_t r = blockIdx.x;
     const uint32_t ng = p.ne0 / 8;
     float v[GPT][8];
     float s0 = 0.0f, s1 = 0.0f, mx = 0.0f;
@@ -559,8 +611,8 @@ __global__ __launch_bounds__(NTH) void k_wide_prep(const WidePrep p)
     }
     if (tid == 0) p.xs[r] = ldexpf(1.0f, -sh);
     const uint64_t nsub = p.ne0 / 32, nsb = p.ne0 / 256;
-    uint8_t *At = p.A + (uint64_t)(r >> 4) * nsub * WIDE_SUB + (r & 15) * 16;
-    uint8_t *St = p.S + (uint64_t)(r >> 4) * nsb * 1024 + (r & 15) * 16;
+    uint8_t *At = p.A + (uint64_t)(r >> 4) * nsub * WIDE_SUB + (r & 15) * 128;
+    uint8_t *St = p.S + (uint64_t)(r >> 4) * nsb * 1024 + (r & 15) * 64;
 #pragma unroll
     for (int i = 0; i < GPT; i++) {
         const uint32_t q = tid + i * NTH, s = q >> 2, g = q & 3;
@@ -580,9 +632,9 @@ __global__ __launch_bounds__(NTH) void k_wide_prep(const WidePrep p)
         const _Float16 p0 = (_Float16)sum, p1 = (_Float16)(sum - (float)p0);
         const _Float16 p2 = (_Float16)((sum - (float)p0) - (float)p1);
         if (q < ng) {
-            *(v8h *)(At + (uint64_t)s * WIDE_SUB + g * 256) = hi;
-            *(v8h *)(At + (uint64_t)s * WIDE_SUB + 1024 + g * 256) = lo;
-            if (g < 3) *(_Float16 *)(St + (uint64_t)(s >> 3) * 1024 + g * 256 + (s & 7) * 2) = g == 0 ? p0 : g == 1 ? p1 : p2;
+            *(v8h *)(At + (uint64_t)s * WIDE_SUB + g * 16) = hi;
+            *(v8h *)(At + (uint64_t)s * WIDE_SUB + 64 + g * 16) = lo;
+            if (p.S && g < 3) *(_Float16 *)(St + (uint64_t)(s >> 3) * 1024 + g * 16 + (s & 7) * 2) = g == 0 ? p0 : g == 1 ? p1 : p2;
         }
     }
 }
@@ -647,7 +699,7 @@ extern "C" int qgpu_wide_supports(const qgpu_tensor *W)
 
 static bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-extern "C" int qgpu_wide_prepare(qgpu_wide *w, const qgpu_act *act, int n, uint64_t ne0)
+extern "C" int qgpu_wide_prepare(qgpu_wide *w, const qgpu_act *act, int n, uint64_t ne0, int sums)
 {
     int rc = qg::ensure_init();
     if (rc) return rc;
@@ -656,7 +708,7 @@ extern "C" int qgpu_wide_prepare(qgpu_wide *w, const qgpu_act *act, int n, uint6
     WidePrep p = {};
     p.x = act->x; p.ldx = act->ldx; p.y = act->y; p.ldy = act->ldy; p.w = act->w; p.w2 = act->w2;
     p.M = (uint32_t)n; p.ne0 = (uint32_t)ne0; p.seg = (uint32_t)ne0; p.eps = act->eps;
-    p.A = w->A; p.S = w->S; p.xs = w->xs;
+    p.A = w->A; p.S = sums ? w->S : nullptr; p.xs = w->xs;
     int kind = act->kind;
     switch (kind) {
     case QGPU_ACT_COPY: break;
@@ -673,11 +725,10 @@ extern "C" int qgpu_wide_prepare(qgpu_wide *w, const qgpu_act *act, int n, uint6
     default: return QGPU_E_ARG;
     }
     if (!al16(p.x) || p.ldx % 4 || (p.y && (!al16(p.y) || p.ldy % 4)) || !al16(p.w) || !al16(p.w2)) return QGPU_E_ARG;
-    // whole groups of 8 tiles (one per XCD); the blocks past the last token exit
-    const dim3 grid((unsigned)((n + 127) / 128 * 128));
+    const dim3 grid((unsigned)n);
 #define WP(KD, G, N) hipLaunchKernelGGL((k_wide_prep<KD, G, N>), grid, dim3(N), 0, qg::stream, p)
 #define WPK(KD) do { if (ne0 <= 3 * 2048) WP(KD, 3, 256); else if (ne0 <= 5 * 2048) WP(KD, 5, 256); \
-                     else if (ne0 <= 9 * 2048) WP(KD, 9, 256); else WP(KD, 8, 1024); } while (0)
+                     else if (ne0 <= 3 * 8192) WP(KD, 3, 1024); else WP(KD, 8, 1024); } while (0)
     switch (kind) {
     case QGPU_ACT_COPY: WPK(QGPU_ACT_COPY); break;
     case QGPU_ACT_RMSNORM: WPK(QGPU_ACT_RMSNORM); break;
@@ -695,13 +746,14 @@ template <int MTL>
 static int wide_launch(int type, WideArgs &a)
 {
     a.mblk = (a.M + MTL * 16 - 1) / (MTL * 16);
-    uint32_t tiles = 0;
+    uint64_t tiles = 0;
     for (int j = 0; j < a.n_mat; j++) {
-        a.m[j].tile0 = tiles;
-        tiles += (a.m[j].rows + WIDE_N - 1) / WIDE_N;
+        a.m[j].tile0 = (uint32_t)tiles;
+        if (!a.pair || !j) tiles += (a.m[j].rows + (a.pair ? WIDE_N / 2 : WIDE_N) - 1) / (a.pair ? WIDE_N / 2 : WIDE_N);
     }
     tiles *= a.mblk;
-    a.U = tiles * a.nsb;
+    if (tiles * a.nsb >= 0xFFFFFFFFull) return QGPU_E_RANGE;
+    a.U = (uint32_t)tiles * a.nsb;
     a.G = a.U < WIDE_MAXG ? a.U : WIDE_MAXG;
 #define WG(F) hipLaunchKernelGGL((k_wide_gemm<F, MTL>), dim3(a.G), dim3(256), 0, qg::stream, a)
     switch (type) {
@@ -714,9 +766,30 @@ static int wide_launch(int type, WideArgs &a)
     }
 #undef WG
     QG_LAUNCH_CHECK();
-    hipLaunchKernelGGL((k_wide_fix<MTL>), dim3(tiles, 4), dim3(256), 0, qg::stream, a);
+    hipLaunchKernelGGL((k_wide_fix<MTL>), dim3((unsigned)tiles, MTL), dim3(256), 0, qg::stream, a);
     QG_LAUNCH_CHECK();
     return QGPU_OK;
+}
+
+static void wide_mat(WideMat &m, const qgpu_tensor *W, float *out, uint64_t ldo)
+{
+    m.W = (const uint8_t *)W->data;
+    m.out = out;
+    m.ldo = ldo;
+    m.rows = (uint32_t)W->ne1;
+    m.nt16 = (uint32_t)((W->ne1 + 15) / 16);
+}
+
+static int wide_go(qgpu_wide *w, int type, uint64_t ne0, int n, WideArgs &a)
+{
+    a.nsb = (uint32_t)(ne0 / 256);
+    a.M = (uint32_t)n;
+    a.A = w->A; a.S = w->S; a.xs = w->xs; a.piece = w->piece;
+    // tokens per block by the tokens of the call: a block's decode work does not shrink with its tokens, so the
+    // smallest tile that holds them all, at most 128 (Q6_K, Q8_0: 64, their records take more registers)
+    const bool narrow = type == T_Q6_K || type == T_Q8_0;
+    const int mtl = n <= 32 ? 2 : (n <= 64 || narrow) ? 4 : 8;
+    return mtl == 2 ? wide_launch<2>(type, a) : mtl == 4 ? wide_launch<4>(type, a) : wide_launch<8>(type, a);
 }
 
 extern "C" int qgpu_wide_gemm(qgpu_wide *w, const qgpu_tensor *const *Ws, int n_mat, int n, float *const *outs,
@@ -734,25 +807,34 @@ extern "C" int qgpu_wide_gemm(qgpu_wide *w, const qgpu_tensor *const *Ws, int n_
     for (int j0 = 0; j0 < n_mat; j0++) {
         if (done >> j0 & 1) continue;
         WideArgs a = {};
-        a.nsb = (uint32_t)(Ws[0]->ne0 / 256);
-        a.M = (uint32_t)n;
         a.accum = (flags & QGPU_GEMV_ACCUM) != 0;
-        a.A = w->A; a.S = w->S; a.xs = w->xs; a.piece = w->piece;
         const int type = Ws[j0]->type;
         for (int j = j0; j < n_mat; j++) {
             if (Ws[j]->type != type) continue;
             done |= 1u << j;
-            WideMat &m = a.m[a.n_mat++];
-            m.W = (const uint8_t *)Ws[j]->data;
-            m.out = outs[j];
-            m.ldo = ldos[j];
-            m.rows = (uint32_t)Ws[j]->ne1;
-            m.nt16 = (uint32_t)((Ws[j]->ne1 + 15) / 16);
+            wide_mat(a.m[a.n_mat++], Ws[j], outs[j], ldos[j]);
         }
-        const bool narrow = type == T_Q6_K || type == T_Q8_0;   // their records take more registers: 64 tokens at most
-        const int mtl = n <= 32 ? 2 : (n <= 64 || narrow) ? 4 : 8;
-        rc = mtl == 2 ? wide_launch<2>(type, a) : mtl == 4 ? wide_launch<4>(type, a) : wide_launch<8>(type, a);
+        rc = wide_go(w, type, Ws[0]->ne0, n, a);
         if (rc) return rc;
     }
     return QGPU_OK;
+}
+
+// silu(gate) * up in the product's epilogue: a block holds the same rows of both matrices, so one fp32 value
+// per pair is written and read back instead of two.
+extern "C" int qgpu_wide_gemm_silu(qgpu_wide *w, const qgpu_tensor *gate, const qgpu_tensor *up, int n, float *out,
+                                   uint64_t ldo)
+{
+    int rc = qg::ensure_init();
+    if (rc) return rc;
+    if (!w || !gate || !up || !out || n < 1 || n > w->rows || gate->ne0 != up->ne0 || gate->ne1 != up->ne1 ||
+        gate->ne0 > w->max_k || ldo < gate->ne1)
+        return QGPU_E_ARG;
+    if (!gate->packed || !up->packed || gate->type != up->type) return QGPU_E_TYPE;
+    WideArgs a = {};
+    a.n_mat = 2;
+    a.pair = 1;
+    wide_mat(a.m[0], gate, out, ldo);
+    wide_mat(a.m[1], up, out, ldo);
+    return wide_go(w, gate->type, gate->ne0, n, a);
 }

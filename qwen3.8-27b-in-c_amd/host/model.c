@@ -1224,13 +1224,21 @@ void gdn_layer(qwen_model_t *m, qwen_layer_t *L, pool_t *pool)
  * It leaves what the tokens after it read: the KV caches (the MTP layer's too), the GDN states (in
  * ring slot cur) and nothing else; prefill_dev runs the prompt's last batch on the ordinary path, so
  * logits, hidden rows and rollback states are those of a batch as before. */
+static void wide_prepare(qwen_model_t *m, const qgpu_act *act, uint32_t M, const qgpu_tensor *const *W, int n_mat)
+{
+    int sums = 0, t;
+    uint64_t ne0 = 0, ne1;
+    for (int i = 0; i < n_mat; i++) {
+        K(qgpu_tensor_shape(W[i], &t, &ne0, &ne1));
+        sums |= t == GGML_Q4_K || t == GGML_Q5_K;
+    }
+    K(qgpu_wide_prepare(m->gpu->wide, act, (int)M, ne0, sums));
+}
+
 static void wide_mul(qwen_model_t *m, const qgpu_act *act, uint32_t M, const qgpu_tensor *const *W, int n_mat,
                      float *const *outs, const uint64_t *ld, int flags)
 {
-    int t;
-    uint64_t ne0 = 0, ne1;
-    K(qgpu_tensor_shape(W[0], &t, &ne0, &ne1));
-    K(qgpu_wide_prepare(m->gpu->wide, act, (int)M, ne0));
+    wide_prepare(m, act, M, W, n_mat);
     K(qgpu_wide_gemm(m->gpu->wide, W, n_mat, (int)M, outs, ld, flags));
 }
 
@@ -1247,12 +1255,21 @@ static void wide_ffn(qwen_model_t *m, const glayer_t *D, uint32_t M)
     qwen_gpu_t *g = m->gpu;
     const uint64_t E = m->dims.n_embd, F = m->dims.n_ff;
     const qgpu_tensor *W[2] = { D->ffn_gate, D->ffn_up };
-    float *outs[2] = { g->wa, g->wb };
-    const uint64_t ld[2] = { F, F };
     const qgpu_act an = act_norm(g->wx, E, D->post_norm, m->cfg.rms_norm_eps, NULL, 0);
-    wide_mul(m, &an, M, W, 2, outs, ld, 0);
-    qgpu_act sm = act_rows(QGPU_ACT_SILU_MUL, g->wa, F);
-    sm.y = g->wb; sm.ldy = F;
+    int tg, tu;
+    uint64_t n0, n1;
+    qgpu_act sm;
+    if (!qgpu_tensor_shape(D->ffn_gate, &tg, &n0, &n1) && !qgpu_tensor_shape(D->ffn_up, &tu, &n0, &n1) && tg == tu) {
+        wide_prepare(m, &an, M, W, 2);
+        K(qgpu_wide_gemm_silu(g->wide, D->ffn_gate, D->ffn_up, (int)M, g->wa, F));
+        sm = act_rows(QGPU_ACT_COPY, g->wa, F);
+    } else {
+        float *outs[2] = { g->wa, g->wb };
+        const uint64_t ld[2] = { F, F };
+        wide_mul(m, &an, M, W, 2, outs, ld, 0);
+        sm = act_rows(QGPU_ACT_SILU_MUL, g->wa, F);
+        sm.y = g->wb; sm.ldy = F;
+    }
     wide_mul(m, &sm, M, (const qgpu_tensor *const *)&D->ffn_down, 1, &g->wx, &E, QGPU_GEMV_ACCUM);
 }
 

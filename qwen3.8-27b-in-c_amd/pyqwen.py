@@ -324,7 +324,8 @@ class GpuLib:
             "qgpu_spec_accept_anchor": [U32P, U32P, i32, i32, i32, i32, ctypes.POINTER(i32), ctypes.POINTER(i32),
                                         i32, U32P, F32P, u64, i32, F32P, U32P, U32P],
             "qgpu_wide_create": [i32, u64, i32, i32, i32, i32, ctypes.POINTER(vp)], "qgpu_wide_free": [vp],
-            "qgpu_wide_supports": [vp], "qgpu_wide_prepare": [vp, ctypes.POINTER(Act), i32, u64],
+            "qgpu_wide_supports": [vp], "qgpu_wide_prepare": [vp, ctypes.POINTER(Act), i32, u64, i32],
+            "qgpu_wide_gemm_silu": [vp, vp, vp, i32, F32P, u64],
             "qgpu_wide_gemm": [vp, ctypes.POINTER(vp), i32, i32, ctypes.POINTER(F32P), ctypes.POINTER(u64), i32],
             "qgpu_wide_attn": [vp, F32P, u64, F32P, F32P, i32, i32, i32, i32, i32, F32P, u64],
             "qgpu_wide_gdn": [vp, F32P, u64, i32, F32P, F32P, F32P, F32P, F32P, u64, F32P, F32P, F32P, F32P, i32,

@@ -61,7 +61,7 @@ def test_wide_gemm_vs_fp64(gpu, fmt, ne0, ne1, n):
     T, xb, ob = gpu.tensor(W, t, ne0, ne1), gpu.put(x), gpu.put(np.full((n + 1) * ne1, 3.0, np.float32))
     with workspace(gpu, n, ne0) as w:
         a = copy_act(xb, ne0)
-        gpu.ok(gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), n, ne0))
+        gpu.ok(gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), n, ne0, 1))
         gemm(gpu, w, [T], [ob], n)
         got = ob.download(np.float32).reshape(n + 1, ne1)
         assert (got[n] == 3.0).all()                                  # rows past the call
@@ -84,7 +84,7 @@ def test_wide_gemm_groups_formats(gpu):
     xb, outs = gpu.put(x), [gpu.buf(n * r * 4) for _, r in mats]
     with workspace(gpu, 128, ne0) as w:
         a = copy_act(xb, ne0)
-        gpu.ok(gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), n, ne0))
+        gpu.ok(gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), n, ne0, 1))
         gemm(gpu, w, Ts, outs, n)
         for W, (t, r), o in zip(Ws, mats, outs):
             ref = x.astype(np.float64) @ O.dequant_rows(t, W, ne0, r).reshape(r, ne0).astype(np.float64).T
@@ -93,7 +93,32 @@ def test_wide_gemm_groups_formats(gpu):
         T.close()
 
 
-@pytest.mark.parametrize("ne0", [256, 6144, 6400, 17408, 18688])
+@pytest.mark.parametrize("t", [23, 13, 8])
+@pytest.mark.parametrize("ne0,ne1,n", [(256, 16, 3), (512, 400, 40), (2560, 1168, 200)])
+def test_wide_gemm_silu(gpu, t, ne0, ne1, n):
+    """silu(gate x) * (up x) from the product, rows off the 128-row halves of its blocks"""
+    host = host_lib()
+    x = host.synth_normal(n * ne0, 8, 8).reshape(n, ne0)
+    Ws = [host.synth_matrix(t, ne0, ne1, 12, i, 0.02) for i in range(2)]
+    g, u = (x.astype(np.float64) @ O.dequant_rows(t, W, ne0, ne1).reshape(ne1, ne0).astype(np.float64).T for W in Ws)
+    Ts = [gpu.tensor(W, t, ne0, ne1) for W in Ws]
+    xb, ob = gpu.put(x), gpu.put(np.full((n + 1) * ne1, 3.0, np.float32))
+    with workspace(gpu, n, ne0) as w:
+        a = copy_act(xb, ne0)
+        gpu.ok(gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), n, ne0, 1))
+        for _ in range(2):
+            gpu.ok(gpu.L.qgpu_wide_gemm_silu(w, Ts[0].h, Ts[1].h, n, ob.f32(), ne1))
+        got = ob.download(np.float32).reshape(n + 1, ne1)
+        F = gpu.tensor(host.synth_matrix(14, ne0, ne1, 1, 1, 0.02), 14, ne0, ne1)
+        assert gpu.L.qgpu_wide_gemm_silu(w, Ts[0].h, F.h, n, ob.f32(), ne1) == -2
+        F.close()
+    assert (got[n] == 3.0).all()
+    assert norm_err(got[:n], g / (1 + np.exp(-g)) * u) < 2e-6        # WIDE_TOL in each factor
+    for T in Ts:
+        T.close()
+
+
+@pytest.mark.parametrize("ne0", [256, 6144, 6400, 17408, 24576, 24832])
 @pytest.mark.parametrize("kind", ["rmsnorm", "cat", "silu", "gated"])
 def test_wide_prepare_kinds(gpu, kind, ne0):
     """each activation transform, at the column counts where the launch shape changes"""
@@ -123,7 +148,7 @@ def test_wide_prepare_kinds(gpu, kind, ne0):
     W = host.synth_matrix(8, ne0, ne1, 5, 6, 0.02)
     T, ob = gpu.tensor(W, 8, ne0, ne1), gpu.buf(n * ne1 * 4)
     with workspace(gpu, n, ne0) as w:
-        gpu.ok(gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), n, ne0))
+        gpu.ok(gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), n, ne0, 1))
         gemm(gpu, w, [T], [ob], n)
         ref = v @ O.dequant_rows(8, W, ne0, ne1).reshape(ne1, ne0).astype(np.float64).T
         assert norm_err(ob.download(np.float32).reshape(n, ne1), ref) < 2e-6   # WIDE_TOL and the transform's own fp32 steps
@@ -138,10 +163,10 @@ def test_wide_rejects(gpu):
     assert gpu.L.qgpu_wide_supports(T.h) == 1 and gpu.L.qgpu_wide_supports(F.h) == 0
     with workspace(gpu, 128, 512) as w:
         a = copy_act(xb, 512)
-        assert gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), 129, 512) == -1
-        assert gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), 8, 768) == -1
+        assert gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), 129, 512, 1) == -1
+        assert gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), 8, 768, 1) == -1
         a.ldx = 514
-        assert gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), 8, 512) == -1
+        assert gpu.L.qgpu_wide_prepare(w, ctypes.byref(a), 8, 512, 1) == -1
         h, o, ld = (ctypes.c_void_p * 1)(F.h), (pyqwen.F32P * 1)(ob.f32()), (ctypes.c_uint64 * 1)(16)
         assert gpu.L.qgpu_wide_gemm(w, h, 1, 8, o, ld, 0) == -2
         assert gpu.L.qgpu_wide_attn(w, xb.f32(), 512, xb.f32(), xb.f32(), 0, 1, 1, 1, 256, ob.f32(), 256) == -1
