@@ -100,7 +100,9 @@ extern "C" int qgpu_malloc(void **p, size_t bytes)
     int rc = qg::ensure_init();
     if (rc) return rc;
     if (!p) return QGPU_E_ARG;
-    return qg::check(hipMalloc(p, bytes ? bytes : 1));
+    const hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+    if (e != hipSuccess) (void)hipGetLastError();        // reported here, not again by the next launch
+    return qg::check(e);
 }
 
 // Work queued on the library stream may still read the allocation: drain the

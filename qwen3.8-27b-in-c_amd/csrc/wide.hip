@@ -219,7 +219,9 @@ typedef __attribute__((address_space(3))) void *lptr_t;
 // (55% of their cycles at 1992 tokens) beside the multiply-adds and decoding on the vector units (49%).
 // Loads take scalar offsets from buffer resources, the next quants the registers of the ones just
 // decoded, and a row tile's multiply-adds run beside the next tile's products: 256 registers hold it, two
-// waves per SIMD.  5120 -> 34816 at 1992 / 256 tokens 1537 / 231 -> 1440 / 208 us, 17408 -> 5120 765 /
+// waves per SIMD.  Power bounds it too: with zero activations the same cycles take 1.10 ms instead of 1.40.
+// (v_mfma_f32_32x32x16_f16 halves the header and scale work: 6% less time for a 33-token prompt, 3% more for
+// 1999 tokens.)  5120 -> 34816 at 1992 / 256 tokens 1537 / 231 -> 1440 / 208 us, 17408 -> 5120 765 /
 // 140 -> 708 / 133 us, against per-lane addresses, copies of the next quants and no such overlap.
 template <int FMT, int MTL>
 __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
@@ -647,9 +649,9 @@ extern "C" int qgpu_wide_free(qgpu_wide *w)
     (void)hipFree(w->A);
     (void)hipFree(w->S);
     (void)hipFree(w->xs);
+    if (w->y != w->piece) (void)hipFree(w->y);
     (void)hipFree(w->piece);
     (void)hipFree(w->kv);
-    (void)hipFree(w->y);
     (void)hipFree(w->gate);
     delete w;
     return QGPU_OK;
@@ -678,13 +680,19 @@ extern "C" int qgpu_wide_create(int max_rows, uint64_t max_k, int n_ctx, int n_k
     if (e == hipSuccess && n_ctx && n_kv) e = hipMalloc((void **)&w->kv, ((size_t)n_ctx + 31) / 32 * n_kv * 65536);
     w->gdn_heads = n_k + 3 * n_v;
     w->gdn_chan = 2 * n_k + n_v;
-    if (e == hipSuccess && n_k && n_v) e = hipMalloc((void **)&w->y, (size_t)w->rows * w->gdn_chan * 128 * sizeof(float));
+    // the recurrence's inputs live between two products: in the pieces' memory where they fit
+    const size_t yb = (size_t)w->rows * w->gdn_chan * 128 * sizeof(float);
+    if (e == hipSuccess && n_k && n_v) {
+        if (yb <= pb) w->y = w->piece;
+        else e = hipMalloc((void **)&w->y, yb);
+    }
     if (e == hipSuccess && n_k && n_v) e = hipMalloc((void **)&w->gate, (size_t)w->rows * w->gdn_heads * sizeof(float));
     // rows past a call's tokens are multiplied too and their results dropped; the fourth part of the sums is 0
     if (e == hipSuccess) e = hipMemsetAsync(w->A, 0, (size_t)w->rows * max_k * 4, qg::stream);
     if (e == hipSuccess) e = hipMemsetAsync(w->S, 0, sb, qg::stream);
     if (e == hipSuccess) e = hipMemsetAsync(w->xs, 0, xb, qg::stream);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         qgpu_wide_free(w);
         return (int)e;
     }

@@ -27,9 +27,9 @@
 #define MAXB  SPEC_MAX_B
 #define WIDE_ROWS 2048              /* prompt tokens per wide chunk at most (a multiple of 8) */
 /* Prompt tokens before the last batch from which the wide path is taken.  Measured at the 27B layer shapes, 8
- * layers, a prompt's ingestion: 16 such tokens 2.67 ms in batches of 8 and 2.72 ms wide (mixed formats
- * 2.52 and 2.59), 24 tokens 3.62 and 2.74 ms (3.36 and 2.60). */
-#define WIDE_MIN  24
+ * layers, a prompt's ingestion: 16 such tokens 2.71 ms in batches of 8 and 2.53 ms wide (mixed formats 2.51
+ * and 2.38), 24 tokens 3.61 and 2.51 ms; 8 tokens, one batch either way, 1.76 and 2.67 ms. */
+#define WIDE_MIN  16
 
 double qwen_prof_embed, qwen_prof_gdn, qwen_prof_attn, qwen_prof_head;
 uint64_t qwen_prof_calls;
@@ -318,36 +318,54 @@ static int upload_layer(qwen_gpu_t *g, const source_t *src, const qwen_layer_t *
 }
 
 /* workspace of the wide prompt path, when every matrix it multiplies runs on the matrix cores */
-static int wide_init(qwen_model_t *m)
+static void wide_init(qwen_model_t *m)
 {
     qwen_gpu_t *g = m->gpu;
     const qwen_dims_t *d = &m->dims;
     const uint64_t E = d->n_embd, F = d->n_ff, hd = (uint64_t)d->n_head * d->head_dim;
+    int apart = 0;                            /* a layer's gate and up differ in format: both are written out */
     for (uint32_t il = 0; il <= d->n_layer; il++) {
         const glayer_t *D = il < d->n_layer ? &g->L[il] : &g->mtp;
         const qgpu_tensor *W[] = { D->ffn_gate, D->ffn_up, D->ffn_down, D->rec ? D->wqkv : D->q,
                                    D->rec ? D->wgate : D->k, D->rec ? D->beta : D->v, D->rec ? D->alpha : D->o,
                                    D->rec ? D->ssm_out : D->o };
         for (size_t i = 0; i < sizeof W / sizeof *W; i++)
-            if (!qgpu_wide_supports(W[i])) return 0;
+            if (!qgpu_wide_supports(W[i])) return;
+        int tg, tu;
+        uint64_t n0, n1;
+        if (qgpu_tensor_shape(D->ffn_gate, &tg, &n0, &n1) || qgpu_tensor_shape(D->ffn_up, &tu, &n0, &n1)) return;
+        if (tg != tu) apart = 1;
     }
-    if (!qgpu_wide_supports(g->eh_proj) || d->n_v_heads % d->n_k_heads) return 0;
+    if (!qgpu_wide_supports(g->eh_proj) || d->n_v_heads % d->n_k_heads) return;
     uint64_t K = F > 2 * E ? F : 2 * E;
     if (g->A > K) K = g->A;
     const uint32_t R = m->n_ctx < WIDE_ROWS ? (m->n_ctx + 7) / 8 * 8 : WIDE_ROWS;
-    if (qgpu_wide_create((int)R, K, (int)m->n_ctx, (int)d->n_kv_head, (int)d->n_k_heads, (int)d->n_v_heads, &g->wide))
-        return -1;
-    g->w_rows = R;
-    const uint64_t B2 = F > E ? F : E, wb = B2 > d->d_inner ? B2 : d->d_inner;
+    const uint64_t B2 = apart && F > E ? F : E, wb = B2 > d->d_inner ? B2 : d->d_inner, nv = d->n_v_heads;
     uint64_t wa = d->conv_dim > 2 * hd ? d->conv_dim : 2 * hd;
     if (F > wa) wa = F;
     if (E > wa) wa = E;
-#define AL(p, n) do { if (!((p) = dalloc(g, (n) * sizeof(*(p))))) return -1; } while (0)
-    AL(g->w_tok, R); AL(g->wx, R * E); AL(g->wa, R * wa); AL(g->wb, R * wb); AL(g->wo, R * g->A);
-    AL(g->wk, R * g->kvrow); AL(g->wv, R * g->kvrow);
-    AL(g->wbeta, R * (uint64_t)d->n_v_heads); AL(g->walpha, R * (uint64_t)d->n_v_heads);
-#undef AL
-    return 0;
+    /* one block of fp32 rows, each array a multiple of 16 bytes (E, F, kvrow, A and the heads of 128 are) */
+    const uint64_t per = E + wa + wb + g->A + 2 * g->kvrow + 2 * ((nv + 3) & ~3ull) + 4;
+    if (qgpu_wide_create((int)R, K, (int)m->n_ctx, (int)d->n_kv_head, (int)d->n_k_heads, (int)nv, &g->wide)) {
+        g->wide = NULL;                       /* no memory for it: prompts go in batches of 8 */
+        return;
+    }
+    float *p = dalloc(g, R * per * sizeof(float));
+    if (!p) {
+        qgpu_wide_free(g->wide);
+        g->wide = NULL;
+        return;
+    }
+    g->w_rows = R;
+    g->wx = p; p += R * E;
+    g->wa = p; p += R * wa;
+    g->wb = p; p += R * wb;
+    g->wo = p; p += R * g->A;
+    g->wk = p; p += R * g->kvrow;
+    g->wv = p; p += R * g->kvrow;
+    g->wbeta = p; p += R * ((nv + 3) & ~3ull);
+    g->walpha = p; p += R * ((nv + 3) & ~3ull);
+    g->w_tok = (uint32_t *)p;
 }
 
 static int model_load(qwen_model_t *m, const source_t *src, uint32_t n_ctx)
@@ -525,7 +543,8 @@ static int model_load(qwen_model_t *m, const source_t *src, uint32_t n_ctx)
               qgpu_memcpy_h2d(g->rope_sin, sn, (size_t)n_ctx * half * sizeof(float)));
     m->rope_cos = cs;                          /* host copies (reference field names) */
     m->rope_sin = sn;
-    if (rc || qgpu_attn_reserve((int)n_ctx, (int)d->n_kv_head) || wide_init(m)) return -1;
+    if (rc || qgpu_attn_reserve((int)n_ctx, (int)d->n_kv_head)) return -1;
+    wide_init(m);
     for (int b = 1; b <= QGPU_MAX_B; b++)
         g->att_split[b] = qgpu_attn_split_bound((int)n_ctx, b, (int)d->n_head, (int)d->n_kv_head);
     /* host-side fields, laid out as the reference's arenas (model.c:166-230) */
