@@ -445,62 +445,57 @@ __global__ __launch_bounds__(256, 2) void k_wide_gemm(const WideArgs a)
     }
 }
 
-// Adds the pieces of the tiles that several blocks computed, in block order: block (tile, row tile mt),
-// the product kernel's lanes and registers, so pieces are written and read in whole lines, four at a time
-// (17408 -> 5120 at 128 tokens, product and sums, 117 -> 70 us; at 512 199 -> 194 us).  A block's last piece starts at its tile's first unit (slot 1),
-// its first one does not (slot 0).
+// Adds the pieces of the tiles that several blocks computed, in block order: block (tile, row tile mt, weight
+// tile t; with a pair, both its halves), the product kernel's lanes and registers, so pieces are written and
+// read in whole lines, eight at a time: a narrow output of few tokens has up to 26 pieces a tile and few
+// tiles, and is bound by the latency of reading them (all four weight tiles in a block, four pieces at a time:
+// a 33-token prompt 2.51 ms, so 2.37; 129 tokens 3.96 -> 3.86).  A block's last piece starts at its tile's first
+// unit (slot 1), its first one does not (slot 0).
 template <int MTL>
 __global__ __launch_bounds__(256) void k_wide_fix(const WideArgs a)
 {
-    const uint32_t tile = blockIdx.x, mt = blockIdx.y, u0 = tile * a.nsb;
+    const uint32_t tile = blockIdx.x, mt = blockIdx.y, tz = blockIdx.z, u0 = tile * a.nsb;
     const uint32_t ga = unit_block(u0, a.G, a.U), gb = unit_block(u0 + a.nsb - 1, a.G, a.U);
     if (ga == gb) return;
     const uint32_t nt = tile / a.mblk, mb = tile - nt * a.mblk, wv = threadIdx.x >> 6, n = threadIdx.x & 15;
     const uint32_t r0 = (mb * MTL + mt) * 16 + 4 * ((threadIdx.x >> 4) & 3);
     if ((mb * MTL + mt) * 16 >= a.M) return;
     constexpr uint64_t PS = MTL * 16 * WIDE_N;
-    const float *P = a.piece + mt * WIDE_NT * 1024 + threadIdx.x * 4;
-    v4f s[WIDE_NT];
+    auto sum = [&](uint32_t t) {
+        const float *P = a.piece + (mt * WIDE_NT + t) * 1024 + threadIdx.x * 4;
+        v4f s = *(const v4f *)(P + (uint64_t)(2 * ga + 1) * PS);
+        for (uint32_t q = ga + 1; q <= gb; q += 8) {
+            v4f v[8];
 #pragma unroll
-    for (int t = 0; t < WIDE_NT; t++) s[t] = *(const v4f *)(P + (uint64_t)(2 * ga + 1) * PS + t * 1024);
-    for (uint32_t q = ga + 1; q <= gb; q += 4) {
-        v4f v[4][WIDE_NT];
+            for (int k = 0; k < 8; k++) v[k] = *(const v4f *)(P + (uint64_t)(2 * min(q + k, gb)) * PS);
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-#pragma unroll
-            for (int t = 0; t < WIDE_NT; t++) v[k][t] = *(const v4f *)(P + (uint64_t)(2 * min(q + k, gb)) * PS + t * 1024);
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-#pragma unroll
-            for (int t = 0; t < WIDE_NT; t++)
-                if (q + k <= gb) s[t] += v[k][t];
-    }
+            for (int k = 0; k < 8; k++)
+                if (q + k <= gb) s += v[k];
+        }
+        return s;
+    };
     const float4 x4 = *(const float4 *)(a.xs + r0);
     const float xr[4] = { x4.x, x4.y, x4.z, x4.w };
+    const v4f s = sum(tz);
     if (a.pair) {
+        const v4f up = sum(tz + WIDE_NT / 2);
+        const uint32_t c = nt * (WIDE_N / 2) + wv * (WIDE_NT * 8) + 16 * tz + n;
 #pragma unroll
-        for (int t = 0; t < WIDE_NT / 2; t++) {
-            const uint32_t c = nt * (WIDE_N / 2) + wv * (WIDE_NT * 8) + 16 * t + n;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (r0 + i < a.M && c < a.m[0].rows)
-                    a.m[0].out[(uint64_t)(r0 + i) * a.m[0].ldo + c] = silu_w(s[t][i] * xr[i]) * (s[t + WIDE_NT / 2][i] * xr[i]);
-        }
+        for (int i = 0; i < 4; i++)
+            if (r0 + i < a.M && c < a.m[0].rows)
+                a.m[0].out[(uint64_t)(r0 + i) * a.m[0].ldo + c] = silu_w(s[i] * xr[i]) * (up[i] * xr[i]);
         return;
     }
     int j = 0;
     while (j + 1 < a.n_mat && nt >= a.m[j + 1].tile0) j++;
+    const uint32_t c = (nt - a.m[j].tile0) * WIDE_N + wv * (WIDE_NT * 16) + 16 * tz + n;
 #pragma unroll
-    for (int t = 0; t < WIDE_NT; t++) {
-        const uint32_t c = (nt - a.m[j].tile0) * WIDE_N + wv * (WIDE_NT * 16) + 16 * t + n;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (r0 + i < a.M && c < a.m[j].rows) {
-                float *o = a.m[j].out + (uint64_t)(r0 + i) * a.m[j].ldo + c;
-                const float v = s[t][i] * xr[i];
-                *o = a.accum ? *o + v : v;
-            }
-    }
+    for (int i = 0; i < 4; i++)
+        if (r0 + i < a.M && c < a.m[j].rows) {
+            float *o = a.m[j].out + (uint64_t)(r0 + i) * a.m[j].ldo + c;
+            const float v = s[i] * xr[i];
+            *o = a.accum ? *o + v : v;
+        }
 }
 
 // ---------------------------------------------------------------- activation preparation
@@ -774,7 +769,7 @@ static int wide_launch(int type, WideArgs &a)
     }
 #undef WG
     QG_LAUNCH_CHECK();
-    hipLaunchKernelGGL((k_wide_fix<MTL>), dim3((unsigned)tiles, MTL), dim3(256), 0, qg::stream, a);
+    hipLaunchKernelGGL((k_wide_fix<MTL>), dim3((unsigned)tiles, MTL, a.pair ? WIDE_NT / 2 : WIDE_NT), dim3(256), 0, qg::stream, a);
     QG_LAUNCH_CHECK();
     return QGPU_OK;
 }

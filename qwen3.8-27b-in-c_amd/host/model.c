@@ -27,8 +27,8 @@
 #define MAXB  SPEC_MAX_B
 #define WIDE_ROWS 2048              /* prompt tokens per wide chunk at most (a multiple of 8) */
 /* Prompt tokens before the last batch from which the wide path is taken.  Measured at the 27B layer shapes, 8
- * layers, a prompt's ingestion: 16 such tokens 2.71 ms in batches of 8 and 2.53 ms wide (mixed formats 2.51
- * and 2.38), 24 tokens 3.61 and 2.51 ms; 8 tokens, one batch either way, 1.76 and 2.67 ms. */
+ * layers, a prompt's ingestion: 16 such tokens 2.71 ms in batches of 8 and 2.36 ms wide, 24 tokens 3.61 and
+ * 2.37 ms; 8 tokens, one batch either way, 1.76 and 2.67 ms. */
 #define WIDE_MIN  16
 
 double qwen_prof_embed, qwen_prof_gdn, qwen_prof_attn, qwen_prof_head;
